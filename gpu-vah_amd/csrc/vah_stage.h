@@ -22,6 +22,7 @@
 #pragma once
 
 #include "vah_device.h"
+#include "vah_face.h"
 #include "vah_source.h"
 
 namespace vah {
@@ -142,71 +143,19 @@ __device__ __forceinline__ int newton_update(double t, const FaceState &S, doubl
     return bad ? -1 : (int)conv;
 }
 
-// The root a face solve's Newton path ends on, and when the path is known to
-// end there.  With Pi = 0 the function the update zeroes is a quadratic in
-// U = u / sqrt(1 + u^2):
-//     f = U (bL + b (e - PL) / 2) - xM,  e = c0 - U xM
-//       = -(b xM / 2) U^2 + B U - xM,    B = bL + b (c0 - PL) / 2,
-// whose smaller root U* = 2 xM / (B + sqrt(B^2 - 2 b xM^2)) is the physical
-// one (the roots' product is 2 / b = 2 for Ft^2 <= 1, and U < 1 for every
-// finite u).  On 0 <= U <= U_v = B / (b xM), left of the vertex, f is
-// increasing and concave in u, so from a start there every Newton iterate
-// after the first lies between the first update and the root: e, which falls
-// as U grows, stays at or above e(U*) on all of them and u stays in [0, u*].
-// A path whose start lies there, whose first update passed the tests and is
-// clearly positive, and whose root has e(U*) clearly positive, can therefore
-// neither fail nor end anywhere but on the root.
-struct FaceRoot {
-    double u;    // u* (when ok)
-    double B;    // the vertex test: start U0 with U0 * bxM <= B
-    double bxM;
-    bool ok;     // a root in [0, 1) with e(U*) clearly positive
-};
-
-__device__ __forceinline__ FaceRoot face_root(double t, const FaceState &S) {
-    const double Ft2 = S.Ft * S.Ft;
-    const double xM = S.x * S.MBT;
-    const double bL = S.x * S.x * S.M0 - Ft2 * S.PL;
-    const double b = S.x * S.x + Ft2;
-    const double c0 = S.M0 - t * S.Ft * S.M3;
-    FaceRoot r;
-    r.B = bL + 0.5 * b * (c0 - S.PL);
-    r.bxM = b * xM;
-    const double disc = r.B * r.B - 2.0 * b * xM * xM;
-    const double U = fdiv(2.0 * xM, r.B + sqrt_pos(fmax(disc, 0.0)));
-    r.ok = (disc >= 0.0) & (r.B > 0.0) & (U >= 0.0) & (U < 1.0) & (c0 - U * xM > 1.e-12 * fabs(c0));
-    r.u = U * rsqrt(fmax(1.0 - U * U, 1.e-300));
-    return r;
-}
-
-// Both sides of a face solved in one loop (independent iterations, each side
-// stops at its own convergence or failure, at most 10^4 iterations each),
-// from `guess`.  Every pass evaluates both updates and keeps each only while
-// its side is still running, so the two dependency chains interleave and the
-// loop body has no branches.  With ROOT_JUMP a side whose first pass shows
-// that its path must end on the root (face_root) takes the root there and
-// stops: two to three passes fewer, and every decision (which sides fail)
-// is the one the full path makes.  Outputs the signed speed v = u^DIR / u^tau
-// of each side; a failed recovery gives the reference's fallback
-// u = (1,0,0,0), i.e. v = 0.
-template <int DIR, bool ROOT_JUMP>
-__device__ __forceinline__ void face_speeds(double t, double guess, const FaceState &A, const FaceState &B, double &vA,
+// Speeds of both sides of a face by the reference's iteration, in one loop
+// (independent iterations, each side stops at its own convergence or failure,
+// at most 10^4 iterations each), from `guess`.  Every pass evaluates both
+// updates and keeps each only while its side is still running, so the two
+// dependency chains interleave and the loop body has no branches.  Outputs the
+// signed speed v = u^DIR / u^tau of each side; a failed recovery gives the
+// reference's fallback u = (1,0,0,0), i.e. v = 0.
+template <int DIR>
+__device__ __forceinline__ void face_newton(double t, double guess, const FaceState &A, const FaceState &B, double &vA,
                                             double &vB) {
-    // the first pass, outside the loop: both sides start at `guess`
-    double ua, ub;
-    int sa = newton_update(t, A, guess, &ua);
-    int sb = newton_update(t, B, guess, &ub);
-    if (ROOT_JUMP) {
-        const FaceRoot qa = face_root(t, A), qb = face_root(t, B);
-        const double U0 = guess * rsqrt(1.0 + guess * guess);  // the first pass's U
-        const bool ja = (sa == 0) & qa.ok & (U0 * qa.bxM <= qa.B) & (ua >= 1.e-9 * guess);
-        const bool jb = (sb == 0) & qb.ok & (U0 * qb.bxM <= qb.B) & (ub >= 1.e-9 * guess);
-        ua = ja ? qa.u : ua;
-        sa = ja ? 1 : sa;
-        ub = jb ? qb.u : ub;
-        sb = jb ? 1 : sb;
-    }
-    for (int it = 1; it < 10000 && (sa == 0 || sb == 0); ++it) {
+    double ua = guess, ub = guess;
+    int sa = 0, sb = 0;
+    for (int it = 0; it < 10000 && (sa == 0 || sb == 0); ++it) {
         double na, nb;
         const int ta = newton_update(t, A, ua, &na);
         const int tb = newton_update(t, B, ub, &nb);
@@ -225,6 +174,28 @@ __device__ __forceinline__ void face_speeds(double t, double guess, const FaceSt
     };
     vA = speed(A, ua, sa);
     vB = speed(B, ub, sb);
+}
+
+// Speeds of both sides of a face, from the start |u_T|^2 = guess2.  With
+// ROOT_JUMP they come in closed form (vah_face.h) wherever both sides' Newton
+// paths must end on it, which is everywhere but in failing or barely physical
+// cells; a lane where one of them need not runs the iteration.
+template <int DIR, bool ROOT_JUMP, typename R>
+__device__ __forceinline__ void face_speeds(double t, double guess2, const R *qR, const R *qL, double &vR, double &vL) {
+    if (ROOT_JUMP) {
+        const FaceStart s = face_start(guess2);
+        auto side = [&](const R *q, double *v) {
+            return face_speed<DIR>(t, (double)q[TTT] - (double)q[PITT], (double)q[TTX] - (double)q[PITX],
+                                   (double)q[TTY] - (double)q[PITY], (double)q[TTN] - (double)q[PITN], (double)q[PL], s,
+                                   v);
+        };
+        const bool okR = side(qR, &vR), okL = side(qL, &vL);
+        if (okR & okL) return;
+    }
+    auto state = [&](const R *q) {
+        return face_state(t, q[TTT], q[TTX], q[TTY], q[TTN], q[PL], q[PITT], q[PITX], q[PITY], q[PITN]);
+    };
+    face_newton<DIR>(t, sqrt_pos(guess2), state(qR), state(qL), vR, vL);
 }
 
 // ---------------------------------------------------------------------------
@@ -297,20 +268,18 @@ __device__ __forceinline__ void face_flux_from(double t, Guess guess, Load load,
 #pragma unroll
         for (int j = 0; j < 4; ++j) raw[n][j] = load(n, j);
     }
-    // the Newton guess |u_T| (loads of its own) after the stencil loads, so
+    // the Newton guess |u_T|^2 (loads of its own) after the stencil loads, so
     // that one wait covers both
-    const double uT_guess = guess();
+    const double guess2 = guess();
     R qL[NN], qR[NN];
 #pragma unroll
     for (int n = 0; n < NN; ++n) {
         R q0 = (R)raw[n][0], q1 = (R)raw[n][1], q2 = (R)raw[n][2], q3 = (R)raw[n][3];
         face_values(q0, q1, q2, q3, qL[n], qR[n]);
     }
-    // the Newton recovery of both sides runs in double whatever R is
-    FaceState FR = face_state(t, qR[TTT], qR[TTX], qR[TTY], qR[TTN], qR[PL], qR[PITT], qR[PITX], qR[PITY], qR[PITN]);
-    FaceState FL = face_state(t, qL[TTT], qL[TTX], qL[TTY], qL[TTN], qL[PL], qL[PITT], qL[PITX], qL[PITY], qL[PITN]);
+    // the recovery of both sides runs in double whatever R is
     double vR, vL;
-    face_speeds<DIR, ROOT_JUMP>(t, uT_guess, FR, FL, vR, vL);
+    face_speeds<DIR, ROOT_JUMP, R>(t, guess2, qR, qL, vR, vL);
     const double a = fmax(fabs(vL), fabs(vR));
     // (F(qR) + F(qL) - a (qR - qL)) / 2 with F(q) = v q
     const R cR = (R)(0.5 * (vR - a)), cL = (R)(0.5 * (vL + a));
@@ -343,9 +312,10 @@ __device__ __forceinline__ void face_flux(double t, Guess guess, const Buf &q, u
         t, guess, [&](int n, int j) { return ld(q, c + (uint32_t)j * stp - 2u * stp, n * f8); }, emit);
 }
 
-__device__ __forceinline__ double uT_of(const Buf &u, uint32_t f8, uint32_t c) {
+// |u_T|^2 at a cell
+__device__ __forceinline__ double uT2_of(const Buf &u, uint32_t f8, uint32_t c) {
     double ux = ld(u, c, f8), uy = ld(u, c, 2 * f8);
-    return sqrt_pos(fabs(ux * ux + uy * uy));
+    return ux * ux + uy * uy;
 }
 
 // d_i of the pi components entering the axis source of direction DIR
@@ -636,7 +606,7 @@ __device__ __forceinline__ void stage_tile(const StageParams &P, int tile, R (*H
                 const int gi = i0 + fi, gj = j0 + fj;  // interior index of the right cell
                 if (fj < TY && gi <= P.nx && gj < P.ny) {
                     const uint32_t c = (plane + (uint32_t)(gj + 2) * sy + (uint32_t)(gi + 2)) * 8u;
-                    face_flux<1, R, true>(t, [&] { return uT_of(V.ucur, f8, c - 8); }, V.qin, f8, c, 8,
+                    face_flux<1, R, true>(t, [&] { return uT2_of(V.ucur, f8, c - 8); }, V.qin, f8, c, 8,
                                     [&](int n, R h) { Hs[n][tid] = h; });
                 }
             }
@@ -653,7 +623,7 @@ __device__ __forceinline__ void stage_tile(const StageParams &P, int tile, R (*H
                 const int gi = i0 + fi, gj = j0 + fj;
                 if (fj <= TY && gi < P.nx && gj <= P.ny) {
                     const uint32_t c = (plane + (uint32_t)(gj + 2) * sy + (uint32_t)(gi + 2)) * 8u;
-                    face_flux<2, R, true>(t, [&] { return uT_of(V.ucur, f8, c - sy8); }, V.qin, f8, c, sy8,
+                    face_flux<2, R, true>(t, [&] { return uT2_of(V.ucur, f8, c - sy8); }, V.qin, f8, c, sy8,
                                     [&](int n, R h) { Hs[n][tid] = h; });
                 }
             }
@@ -678,13 +648,13 @@ __device__ __forceinline__ void stage_tile(const StageParams &P, int tile, R (*H
 #pragma unroll
                             for (int n = 0; n < NQ; ++n) zr(kk + j - 2, n) = (R)v[n];
                         }
-                        face_flux_from<3, R, true>(t, [&] { return uT_of(V.ucur, f8, s - sz8); },
+                        face_flux_from<3, R, true>(t, [&] { return uT2_of(V.ucur, f8, s - sz8); },
                             [&](int n, int j) {
                                 return j == 0 ? ld(V.qin, s - 2u * sz8, n * f8) : (double)zr(kk + j - 2, n);
                             },
                             [&](int n, R h) { Hz[n][tid] = h; });
                     } else {
-                        face_flux<3, R, true>(t, [&] { return uT_of(V.ucur, f8, s - sz8); }, V.qin, f8, s, sz8,
+                        face_flux<3, R, true>(t, [&] { return uT2_of(V.ucur, f8, s - sz8); }, V.qin, f8, s, sz8,
                                         [&](int n, R h) { Hz[n][tid] = h; });
                     }
                 }
@@ -698,17 +668,17 @@ __device__ __forceinline__ void stage_tile(const StageParams &P, int tile, R (*H
                     double fresh[NQ];
 #pragma unroll
                     for (int n = 0; n < NQ; ++n) fresh[n] = ld(V.qin, s + 2u * sz8, n * f8);
-                    face_flux_from<3, R, true>(t, [&] { return uT_of(V.ucur, f8, s); },
+                    face_flux_from<3, R, true>(t, [&] { return uT2_of(V.ucur, f8, s); },
                         [&](int n, int j) { return j < 3 ? (double)zr(kk - 1 + j, n) : fresh[n]; }, upper);
 #pragma unroll
                     for (int n = 0; n < NQ; ++n) zr(kk + 2, n) = (R)fresh[n];
                 } else {
-                    face_flux<3, R, true>(t, [&] { return uT_of(V.ucur, f8, s); }, V.qin, f8, s + sz8, sz8, upper);
+                    face_flux<3, R, true>(t, [&] { return uT2_of(V.ucur, f8, s); }, V.qin, f8, s + sz8, sz8, upper);
                 }
             }
         } else if (cell_ok) {
             // reference work split: both faces of each direction, Newton guess from this cell
-            const double uTs = uT_of(V.ucur, f8, s);
+            const double uTs = uT2_of(V.ucur, f8, s);
             {
                 R Sa[4];
                 axis_source<1>(axis_pi<1, R>(V.qin, f8, s, 8, P.hx), (R)(ld(V.ucur, s, f8) * iut), Sa);
