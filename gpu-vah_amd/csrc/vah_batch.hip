@@ -603,9 +603,9 @@ int finish_admission(vah_batch *b, int s, const double *dev_in, int has_pl, int 
     hipLaunchKernelGGL(init_event_kernel, dim3(blocks), dim3(256), 0, b->stream, dev_in, has_pl, has_u, has_pi,
                        d->nx, d->ny, d->nz, (long)h.lay.ncx, (long)h.lay.ncx * h.lay.ncy, h.lay.fs, d->t0, b->eos,
                        h.dev.q[0], h.dev.e[0], h.dev.p[0], h.dev.u[0], h.dev.u[1]);
-    hipLaunchKernelGGL(ghost_fill_kernel, dim3(blocks), dim3(256), 0, b->stream, h.dev.q[0], h.dev.e[0], h.dev.p[0],
-                       h.dev.u[0], h.lay.fs, d->nx, d->ny, d->nz, (long)h.lay.ncx, (long)h.lay.ncx * h.lay.ncy,
-                       d->nz > 1 ? 1 : 0);
+    hipLaunchKernelGGL(ghost_fill_kernel, ghost_grid(d->nx, d->ny, d->nz), dim3(256), 0, b->stream, h.dev.q[0],
+                       h.dev.e[0], h.dev.p[0], h.dev.u[0], h.lay.fs, d->nx, d->ny, d->nz, (long)h.lay.ncx,
+                       (long)h.lay.ncx * h.lay.ncy, d->nz > 1 ? 1 : 0, nullptr);
     if (hipGetLastError() != hipSuccess) {
         release_event(b, s);
         return fail(VAH_ERR_HIP, "%s: initial-state launch", who);

@@ -334,11 +334,9 @@ void launch_stage(const LaunchCfg &L, int stage, const StageParams &P) {
 }
 
 int fill_ghosts(vah_ctx *c) {
-    long n = (long)c->lat.nx * c->lat.ny * c->lat.nz;
-    int blocks = (int)((n + 255) / 256);
-    hipLaunchKernelGGL(ghost_fill_kernel, dim3(blocks), dim3(256), 0, c->stream, c->qset[c->qi], c->ebuf[c->ecur],
-                       c->pbuf[c->ecur], c->useq[c->uc], c->fs, c->lat.nx, c->lat.ny, c->lat.nz, (long)c->ncx,
-                       (long)c->ncx * c->ncy, c->lat.nz > 1 ? 1 : 0);
+    hipLaunchKernelGGL(ghost_fill_kernel, ghost_grid(c->lat.nx, c->lat.ny, c->lat.nz), dim3(256), 0, c->stream,
+                       c->qset[c->qi], c->ebuf[c->ecur], c->pbuf[c->ecur], c->useq[c->uc], c->fs, c->lat.nx, c->lat.ny,
+                       c->lat.nz, (long)c->ncx, (long)c->ncx * c->ncy, c->lat.nz > 1 ? 1 : 0, nullptr);
     HIP_TRY(hipGetLastError());
     return VAH_OK;
 }
@@ -608,10 +606,6 @@ int noalloc_setup(int dev, NoallocDevice **out) {
     if (d.rc != VAH_OK) return fail(d.rc, "vah_step_noalloc: set-up on device %d: %s", dev, d.err.c_str());
     *out = &d;
     return VAH_OK;
-}
-
-__global__ void clear_counters_kernel(unsigned int *c) {
-    if (threadIdx.x < 4) c[threadIdx.x] = 0u;
 }
 
 }  // namespace
@@ -973,20 +967,13 @@ int vah_step_noalloc(const vah_lattice *lat, const vah_hydro *hydro, const vah_o
     double *scr = D->scratch;
     unsigned int *cnt = counters ? counters : (unsigned int *)(scr + (size_t)kStageFields * lay.fs);
     hipStream_t stream = (hipStream_t)opt->stream;
-    if (!counters) {
-        // a fill kernel (no memset node when the caller captures the stream)
-        hipLaunchKernelGGL(clear_counters_kernel, dim3(1), dim3(64), 0, stream, cnt);
-        HIP_TRY(hipGetLastError());
-    }
     // zero-gradient ghosts of the inputs (every later input is a stage output,
-    // whose ghosts the stage kernels write)
-    {
-        const long n = lay.interior();
-        hipLaunchKernelGGL(ghost_fill_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, st->q, st->e,
-                           st->p, st->u, lay.fs, lat->nx, lat->ny, lat->nz, (long)lay.ncx,
-                           (long)lay.ncx * lay.ncy, lat->nz > 1 ? 1 : 0);
-        HIP_TRY(hipGetLastError());
-    }
+    // whose ghosts the stage kernels write); the library's own counters are
+    // cleared by the same launch (no memset node when the caller captures)
+    hipLaunchKernelGGL(ghost_fill_kernel, ghost_grid(lat->nx, lat->ny, lat->nz), dim3(256), 0, stream, st->q, st->e,
+                       st->p, st->u, lay.fs, lat->nx, lat->ny, lat->nz, (long)lay.ncx, (long)lay.ncx * lay.ncy,
+                       lat->nz > 1 ? 1 : 0, counters ? nullptr : cnt);
+    HIP_TRY(hipGetLastError());
     const Geometry g = make_geometry(*lat, opt->eta_chunk);
     const LaunchCfg L{g.grid, stream, opt->precision, opt->flux_mode, lat->nz > 1};
     StageParams P = base_params(*lat, *hydro, lay, g, eos, cnt);
