@@ -34,11 +34,10 @@ using namespace vah;
 using vah_host::fail;
 
 namespace vah {
-// one launch function per compiled variant (vah_batch_variant.hip)
-void batch_stage_v16x15b2(const BatchLaunch &, bool, bool, bool);
-void batch_stage_v32x7b2(const BatchLaunch &, bool, bool, bool);
-void batch_stage_v32x7b3(const BatchLaunch &, bool, bool, bool);
-void batch_stage_v16x15b3(const BatchLaunch &, bool, bool, bool);
+// one launch function per compiled tile shape (vah_batch_variant.hip)
+void batch_stage_t16x15(const BatchLaunch &, bool, bool, bool);
+void batch_stage_t8x7(const BatchLaunch &, bool, bool, bool);
+void batch_stage_t16x7(const BatchLaunch &, bool, bool, bool);
 }  // namespace vah
 
 namespace {
@@ -49,17 +48,22 @@ constexpr size_t kAlign = 256;
 
 struct Variant {
     vah_batch_variant info;
+    int waves_per_role;  // of the stage workgroup (vah_stage.h)
     BatchStageFn fn;
 };
 
+// Tile shapes and eta chunks the autotuner chooses from.  64 boost-invariant
+// events of side 101-261 take 0.98 / 1.01 / 1.00 / 1.03 / 1.03 ms per step with
+// them in this order, a few events (whose tiles do not fill the chip) least
+// with the smallest tile, which is the default.
 const Variant kVariants[] = {
-    {{16, 15, 2, 3}, batch_stage_v16x15b2},
-    {{16, 15, 2, 6}, batch_stage_v16x15b2},
-    {{32, 7, 2, 3}, batch_stage_v32x7b2},
-    {{32, 7, 2, 6}, batch_stage_v32x7b2},
-    {{16, 15, 3, 3}, batch_stage_v16x15b3},
-    {{32, 7, 3, 3}, batch_stage_v32x7b3},
+    {{16, 15, kWavesPerSimd, 3}, 4, batch_stage_t16x15},
+    {{8, 7, kWavesPerSimd, 3}, 1, batch_stage_t8x7},
+    {{8, 7, kWavesPerSimd, 6}, 1, batch_stage_t8x7},
+    {{16, 7, kWavesPerSimd, 3}, 2, batch_stage_t16x7},
+    {{16, 7, kWavesPerSimd, 6}, 2, batch_stage_t16x7},
 };
+constexpr int kDefaultVariant = 1;
 constexpr int kNumVariants = (int)(sizeof kVariants / sizeof kVariants[0]);
 
 struct HostEvent {
@@ -279,11 +283,10 @@ int upload_lists(vah_batch *b) {
     return VAH_OK;
 }
 
-// persistent workgroups: the variant's occupancy, at most 2 per CU for 3+1D
-// tiles (their face and eta buffers fill half a CU's LDS)
-int grid_of(const vah_batch *b, bool d3) {
-    const vah_batch_variant &v = kVariants[b->variant].info;
-    int g = b->num_cus * (d3 ? std::min(v.blocks_per_cu, 2) : v.blocks_per_cu);
+// persistent workgroups: as many as the CUs hold at once (4 SIMDs of
+// kWavesPerSimd waves, 2 x waves_per_role waves per workgroup)
+int grid_of(const vah_batch *b) {
+    const int g = b->num_cus * 4 * kWavesPerSimd / (2 * kVariants[b->variant].waves_per_role);
     return std::max(8, g / 8 * 8);
 }
 
@@ -297,8 +300,7 @@ void enqueue_step(vah_batch *b, bool has2, bool has3) {
     L.tiles2 = b->tiles_dev;
     L.tiles3 = b->tiles_dev + b->cap2;
     L.counts = b->counts_dev;
-    L.grid = grid_of(b, false);
-    L.grid3 = grid_of(b, true);
+    L.grid = grid_of(b);
     L.stream = b->stream;
     const bool fp32 = b->opt.precision == VAH_FP32_SPLIT;
     BatchStageFn fn = kVariants[b->variant].fn;
@@ -497,7 +499,7 @@ int vah_batch_create(const vah_batch_options *opt_in, vah_batch **out) {
     b->device = opt.device;
     b->max_events = opt.max_events;
     b->events.resize(opt.max_events);
-    b->variant = opt.variant < 0 ? 0 : opt.variant;
+    b->variant = opt.variant < 0 ? kDefaultVariant : opt.variant;
     b->lists_dirty = true;
     auto cleanup = [&](int code) {
         vah_batch_destroy(b);

@@ -112,11 +112,11 @@ static __global__ void batch_prepare_kernel(const BatchEvent *__restrict__ ev, B
 // One stage over the tile list of one dimensionality.  tiles[w] = (slot,
 // tile index within the event); ntiles[0] / ntiles[1] count the 2+1D / 3+1D
 // lists.  gridDim.x is a multiple of 8 (one share per XCD).
-template <bool D3, bool STAGE2, typename R, int TX, int TY, int BLOCKS>
-__global__ __launch_bounds__(NTHREADS, BLOCKS) void batch_stage_kernel(const BatchStageRec *__restrict__ rec,
-                                                                      const int2 *__restrict__ tiles,
-                                                                      const int *__restrict__ ntiles) {
-    __shared__ StageLds<D3, true, R> lds;
+template <bool D3, bool STAGE2, typename R, int TX, int TY, int NW>
+__global__ __launch_bounds__(128 * NW, kWavesPerSimd) void batch_stage_kernel(const BatchStageRec *__restrict__ rec,
+                                                                             const int2 *__restrict__ tiles,
+                                                                             const int *__restrict__ ntiles) {
+    __shared__ StageLds<D3, R, NW> lds;
     const int n = ntiles[D3 ? 1 : 0];
     const int xcd = (int)(blockIdx.x & 7u), loc = (int)(blockIdx.x >> 3), nloc = (int)(gridDim.x >> 3);
     const int lo = (int)(((long long)n * xcd) >> 3), hi = (int)(((long long)n * (xcd + 1)) >> 3);
@@ -130,10 +130,9 @@ __global__ __launch_bounds__(NTHREADS, BLOCKS) void batch_stage_kernel(const Bat
         const int slot = __builtin_amdgcn_readfirstlane(tr.x);
         const int tile = __builtin_amdgcn_readfirstlane(tr.y);
         const BatchStageRec &r = rec[2 * slot + (STAGE2 ? 1 : 0)];
-        if (r.live != 0) {
-            stage_tile<D3, STAGE2, true, R, TX, TY>(r.P, tile, lds.Hs, lds.Hz, &lds.Zr[0][0][0]);
-            __syncthreads();  // the next tile rewrites the face buffers
-        }
+        // the tile's last barrier frees the LDS, so the face waves go on to the
+        // next tile while the cell waves finish this one
+        if (r.live != 0) stage_tile<D3, STAGE2, R, TX, TY, NW>(r.P, tile, lds);
         if (wn >= hi) break;
         w = wn;
         tr = next;
@@ -176,7 +175,7 @@ struct BatchLaunch {
     const BatchStageRec *rec;
     const int2 *tiles2, *tiles3;  // 2+1D and 3+1D tile lists
     const int *counts;            // [0] 2+1D tiles, [1] 3+1D tiles, [2] active events
-    int grid, grid3;              // persistent workgroups for 2+1D / 3+1D tiles (multiples of 8)
+    int grid;                     // persistent workgroups (a multiple of 8)
     hipStream_t stream;
 };
 

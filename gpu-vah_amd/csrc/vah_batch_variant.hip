@@ -1,6 +1,6 @@
 // vah_batch_variant.hip -- instantiates the persistent batch stage kernels for
-// one tile shape and occupancy target.  Built twice per variant with
-//   -DVAH_BV_TX=<tile x> -DVAH_BV_TY=<tile y> -DVAH_BV_B=<workgroups per CU>
+// one tile shape.  Built twice per shape with
+//   -DVAH_BV_TX=<tile x> -DVAH_BV_TY=<tile y> -DVAH_BV_NW=<waves per role>
 //   -DVAH_BV_FN=<name of the launch function> -DVAH_BV_FN3=<its 3+1D part>
 // and -DVAH_BV_PART=2 (the launch function and the 2+1D kernels) or
 // -DVAH_BV_PART=3 (the 3+1D kernels), so that the two dimensionalities can be
@@ -8,24 +8,19 @@
 // vah_batch.hip lists the builds).
 #include "vah_batch_kernels.h"
 
-#if !defined(VAH_BV_TX) || !defined(VAH_BV_TY) || !defined(VAH_BV_B) || !defined(VAH_BV_FN) || \
+#if !defined(VAH_BV_TX) || !defined(VAH_BV_TY) || !defined(VAH_BV_NW) || !defined(VAH_BV_FN) || \
     !defined(VAH_BV_FN3) || !defined(VAH_BV_PART)
-#error "vah_batch_variant.hip needs VAH_BV_TX, VAH_BV_TY, VAH_BV_B, VAH_BV_FN, VAH_BV_FN3 and VAH_BV_PART"
+#error "vah_batch_variant.hip needs VAH_BV_TX, VAH_BV_TY, VAH_BV_NW, VAH_BV_FN, VAH_BV_FN3 and VAH_BV_PART"
 #endif
 
 namespace vah {
 
 namespace {
 
-// a 3+1D workgroup carries the eta faces in LDS as well (2 x 15 x 256
-// values): at most two fit a CU in double precision
-constexpr int kBlocks3D = VAH_BV_B > 2 ? 2 : VAH_BV_B;
-
 template <bool D3, bool S2, typename R>
 void launch_one(const BatchLaunch &L) {
-    constexpr int B = D3 ? kBlocks3D : VAH_BV_B;
-    hipLaunchKernelGGL((batch_stage_kernel<D3, S2, R, VAH_BV_TX, VAH_BV_TY, B>), dim3(D3 ? L.grid3 : L.grid), dim3(NTHREADS),
-                       0, L.stream, L.rec, D3 ? L.tiles3 : L.tiles2, L.counts);
+    hipLaunchKernelGGL((batch_stage_kernel<D3, S2, R, VAH_BV_TX, VAH_BV_TY, VAH_BV_NW>), dim3(L.grid),
+                       dim3(128 * VAH_BV_NW), 0, L.stream, L.rec, D3 ? L.tiles3 : L.tiles2, L.counts);
 }
 
 template <bool D3, typename R>

@@ -178,21 +178,37 @@ bool lattice_ok(const vah_lattice *l) {
     return l && l->nx > 0 && l->ny > 0 && l->nz > 0 && l->dx > 0 && l->dy > 0 && l->dz > 0 && l->dt > 0;
 }
 
-// Launch geometry of one lattice: 16 x 15 tiles marching kz eta planes.
+// Launch geometry of one lattice: tiles marching kz eta planes.
 struct Geometry {
     int tiles_x, tiles_y, zchunks, kz, nblocks, grid;
 };
 
-Geometry make_geometry(const vah_lattice &lat, int eta_chunk) {
+// Eta planes per workgroup when the caller leaves the choice (opt.eta_chunk 0).
+// A chunk of kz planes solves kz + 1 eta faces per cell and starts by loading
+// three planes of each column, so longer chunks do less work; but a lattice of
+// few tiles then leaves CUs idle.  About 1,024 workgroups (four per CU) run at
+// once.  Measured per pass with kz = 1 / 3 / 6: 53x67x13 (70 tiles) 192 / 281 /
+// 424 us, 101x101x30 (195 tiles) 830 / 775 / 775 us, 201x201x101 (754 tiles)
+// 2.62 / 2.41 / 2.40 ms per step (12: 2.49).
+int choose_eta_chunk(int tiles, int nz) {
+    auto groups = [&](int kz) { return (long)tiles * ((nz + kz - 1) / kz); };
+    if (groups(6) >= 4096) return 6;
+    if (groups(3) >= 1536) return 3;
+    if (groups(2) >= 1536) return 2;
+    return 1;
+}
+
+Geometry make_geometry(const vah_lattice &lat, int flux_mode, int eta_chunk) {
+    const bool shared = flux_mode == VAH_FLUX_SHARED;
+    const int tx = shared ? kTileX : kCellTileX, ty = shared ? kTileY : kCellTileY;
     Geometry g;
-    g.tiles_x = (lat.nx + kTileX - 1) / kTileX;
-    g.tiles_y = (lat.ny + kTileY - 1) / kTileY;
-    // eta planes per workgroup: 3 by default (fastest in a sweep at 201x201x101)
-    const int kz_default = 3;
-    g.kz = lat.nz > 1 ? std::min(eta_chunk > 0 ? eta_chunk : kz_default, lat.nz) : 1;
+    g.tiles_x = (lat.nx + tx - 1) / tx;
+    g.tiles_y = (lat.ny + ty - 1) / ty;
+    const int tiles = g.tiles_x * g.tiles_y;
+    g.kz = lat.nz > 1 ? std::min(eta_chunk > 0 ? eta_chunk : choose_eta_chunk(tiles, lat.nz), lat.nz) : 1;
     g.zchunks = (lat.nz + g.kz - 1) / g.kz;
-    g.nblocks = g.tiles_x * g.tiles_y * g.zchunks;
-    g.grid = g.zchunks * 8 * ((g.tiles_x * g.tiles_y + 7) / 8);  // tile_of_block's grid
+    g.nblocks = tiles * g.zchunks;
+    g.grid = g.zchunks * 8 * ((tiles + 7) / 8);  // tile_of_block's grid
     return g;
 }
 
@@ -308,19 +324,19 @@ LaunchCfg launch_cfg(const vah_ctx *c) {
     return LaunchCfg{c->grid, c->stream, c->opt.precision, c->opt.flux_mode, c->lat.nz > 1};
 }
 
-template <bool D3, bool S2, bool SH, typename R>
+template <bool S2, typename R>
 void launch(const LaunchCfg &L, const StageParams &P) {
-    hipLaunchKernelGGL((stage_kernel<D3, S2, SH, R>), dim3(L.grid), dim3(NTHREADS), 0, L.stream, P);
+    hipLaunchKernelGGL((stage_kernel<false, S2, R>), dim3(L.grid), dim3(128 * kTileWaves), 0, L.stream, P);
 }
 
-template <bool D3, bool S2>
+template <bool S2>
 void launch_variant(const LaunchCfg &L, const StageParams &P) {
     if (L.precision == VAH_FP32_SPLIT)
-        launch<D3, S2, true, float>(L, P);
+        launch<S2, float>(L, P);
     else if (L.flux_mode == VAH_FLUX_SHARED)
-        launch<D3, S2, true, double>(L, P);
+        launch<S2, double>(L, P);
     else
-        launch<D3, S2, false, double>(L, P);
+        hipLaunchKernelGGL((stage_per_cell_kernel<false, S2>), dim3(L.grid), dim3(kCellThreads), 0, L.stream, P);
 }
 
 // 2+1D here; 3+1D in vah_stage3d.hip (compiled with other scheduler settings)
@@ -328,8 +344,8 @@ void launch_stage(const LaunchCfg &L, int stage, const StageParams &P) {
     if (L.d3) {
         launch_stage_3d(StageLaunch{L.grid, L.stream, L.precision, L.flux_mode}, stage, P);
     } else {
-        if (stage == 1) launch_variant<false, false>(L, P);
-        else launch_variant<false, true>(L, P);
+        if (stage == 1) launch_variant<false>(L, P);
+        else launch_variant<true>(L, P);
     }
 }
 
@@ -721,7 +737,7 @@ int vah_create(const vah_lattice *lat, const vah_hydro *hydro, const vah_options
 
     // launch geometry
     {
-        Geometry g = make_geometry(*lat, opt.eta_chunk);
+        Geometry g = make_geometry(*lat, opt.flux_mode, opt.eta_chunk);
         c->tiles_x = g.tiles_x;
         c->tiles_y = g.tiles_y;
         c->kz = g.kz;
@@ -974,7 +990,7 @@ int vah_step_noalloc(const vah_lattice *lat, const vah_hydro *hydro, const vah_o
                        st->p, st->u, lay.fs, lat->nx, lat->ny, lat->nz, (long)lay.ncx, (long)lay.ncx * lay.ncy,
                        lat->nz > 1 ? 1 : 0, counters ? nullptr : cnt);
     HIP_TRY(hipGetLastError());
-    const Geometry g = make_geometry(*lat, opt->eta_chunk);
+    const Geometry g = make_geometry(*lat, opt->flux_mode, opt->eta_chunk);
     const LaunchCfg L{g.grid, stream, opt->precision, opt->flux_mode, lat->nz > 1};
     StageParams P = base_params(*lat, *hydro, lay, g, eos, cnt);
     StepBuffers B;

@@ -24,6 +24,9 @@ struct SrcIn {
     double dxp, dyp, dnp, dxe, dye, dne, dxpl, dypl, dnpl;
 };
 
+__device__ __forceinline__ float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 // R is the arithmetic type of the source terms: double, or float for the
 // split-precision form (the rational fits and the temperature stay double).
 template <typename R, typename QA>
@@ -44,6 +47,10 @@ __device__ __forceinline__ void source_terms(const Eos &E, const SrcIn &in, cons
     const R dkvk = ((dxux - vx * dxut) + (dyuy - vy * dyut) + (dnun - vn * dnut)) * iut;
 
     const R t2 = t * t, it2 = it * it, un2 = un * un, ut2 = ut * ut;
+    // 1/t^2 + (u^eta)^2, contracted here rather than by the compiler: which of
+    // the two squares it fuses depends on the surrounding code, and in float
+    // the shear tensor's cancelling terms make the choice visible
+    const R it2un2 = fused(un, un, it2);
 
     const R dtut = (ut - in.utp) * in.dt_inv, dtux = (ux - in.uxp) * in.dt_inv;
     const R dtuy = (uy - in.uyp) * in.dt_inv, dtun = (un - in.unp) * in.dt_inv;
@@ -71,7 +78,7 @@ __device__ __forceinline__ void source_terms(const Eos &E, const SrcIn &in, cons
     const R sxn = -ut * ux * un * it - R(0.5) * (dxun + dnux * it2) - R(0.5) * (un * dux + ux * dun) + ux * un * th3;
     const R syy = -(dyuy + uy * duy) + (R(1.0) + uy * uy) * th3;
     const R syn = -ut * uy * un * it - R(0.5) * (dyun + dnuy * it2) - R(0.5) * (un * duy + uy * dun) + uy * un * th3;
-    const R snn = -ut * (R(1.0) + R(2.0) * t2 * un2) * it2 * it - dnun * it2 - un * dun + (it2 + un2) * th3;
+    const R snn = -ut * (R(1.0) + R(2.0) * t2 * un2) * it2 * it - dnun * it2 - un * dun + it2un2 * th3;
 
     // longitudinal unit vector z^mu and the transverse / longitudinal split
     const R uTdtuT = ux * dtux + uy * dtuy;
@@ -218,7 +225,7 @@ __device__ __forceinline__ void source_terms(const Eos &E, const SrcIn &in, cons
     const R I4yy = (pity * styT - pixy * sxyT - piyy * syyT - t2 * piyn * synT) + (R(1.0) + uy * uy) * ps2;
     const R I4yn = R(0.5) * ((pity * stnT + pitn * styT) - (pixy * sxnT + pixn * sxyT) - (piyy * synT + piyn * syyT) -
                                t2 * (piyn * snnT + pinn * synT)) + (uy * un) * ps2;
-    const R I4nn = (pitn * stnT - pixn * sxnT - piyn * synT - t2 * pinn * snnT) + (it2 + un2 - z32) * ps2;
+    const R I4nn = (pitn * stnT - pixn * sxnT - piyn * synT - t2 * pinn * snnT) + (it2un2 - z32) * ps2;
 
     // I = I1 - delta_pipi I2 + tau_pipi I4 - lambda_pipi I5 with I2 = thetaT pi, I5 = zDzu pi
     const R c25 = delta_pipi * thetaT + lambda_pipi * zDzu;

@@ -8,15 +8,25 @@
 //   Newton recovery of (e, p, u) at tau + dt, regulation, and the
 //   zero-gradient ghost copies of all outputs (DynamicalVariables.cpp:349-489).
 //
-// Work decomposition.  A workgroup of 256 lanes (4 wave64) owns a 16 x 15
-// tile of cells in (x, y) and marches through KZ consecutive eta planes.
-// Face fluxes are the expensive part (two Newton solves each).  With
-// SHARED, each x or y face of the tile is solved once by one lane, its
-// 15-component flux parked in LDS and read by the two cells that share it;
-// the eta face between planes k and k+1 is solved by the cell's own lane and
-// carried to the next plane in an LDS slot only that lane touches (in
-// registers it would push the kernel into spilling).  Without SHARED every cell solves
-// both of its faces with its own Newton guess, the reference's work split.
+// Work decomposition.  A workgroup owns a TX x TY tile of cells in (x, y) and
+// marches through kz consecutive eta planes.  Its waves have two roles, each
+// with one lane per cell of the tile:
+//   face waves   solve each x, y and eta face of the tile once and leave the
+//                15-component fluxes (and the axis sources, whose pi gradients
+//                are differences of values the face has loaded) in LDS;
+//   cell waves   form the source terms of the plane meanwhile, then add the
+//                fluxes and finish the cell: recovery, regulator, stores.
+// The two halves of a cell's work take about the same time, so they run side
+// by side instead of one after the other, with one exchange per plane.  In a
+// kernel whose every wave did both, a stage of a lattice that does not fill
+// the chip was one long serial chain (28 us at 81x81 and at 261x243), four
+// barriers a plane kept its four waves in step, and its register need (250,
+// two waves per SIMD) was that of the union of both halves.
+// Measured, one step: 81x81 57 -> 20 us, 261x243 56 -> 43 us, 611x587 172 ->
+// 153 us, 101x101x30 296 -> 194 us, 97x89x33 in split precision 336 -> 180 us,
+// 201x201x101 2.55 -> 2.40 ms.
+// VAH_FLUX_PER_CELL keeps the reference's work split in a kernel of its own:
+// every cell solves both of its faces with its own Newton guess.
 // Workgroups are mapped to tiles so that the eight XCDs work through the eta
 // chunks together (tile_of_block).
 #pragma once
@@ -27,23 +37,27 @@
 
 namespace vah {
 
-// workgroups per CU the register allocation is sized for (occupancy target)
-#ifndef VAH_BLOCKS_2D
-#define VAH_BLOCKS_2D 2
-#endif
-#ifndef VAH_BLOCKS_3D
-#define VAH_BLOCKS_3D 2
-#endif
+// Tile of the single-lattice kernels: 8 x 7 cells, one face wave and one cell
+// wave.  Its x faces (9 x 7 = 63) and y faces (8 x 8 = 64) fill a wave, its
+// cells 56 lanes of one.
+constexpr int kTileX = 8;
+constexpr int kTileY = 7;
+constexpr int kTileWaves = 1;  // waves per role
 
-// default tile: 16 x 15 cells (x faces 17 x 15, y faces 16 x 16 fill 255 / 256 lanes)
-constexpr int kTileX = 16;
-constexpr int kTileY = 15;
-constexpr int NTHREADS = 256;
+// The per-cell-flux kernels: 256 lanes, one per cell of a 16 x 16 tile.
+constexpr int kCellTileX = 16;
+constexpr int kCellTileY = 16;
+constexpr int kCellThreads = 256;
 
-// a tile shape fits one workgroup when its cells and both face sets do
-template <int TX, int TY>
+// Waves per SIMD the register allocation is sized for: 512 registers shared by
+// two leave 256 to each.  At three (168 each) the source terms spill and every
+// lattice measured slower (101x101x30: 789 against 1058 us for four steps).
+constexpr int kWavesPerSimd = 2;
+
+// a tile shape fits NW waves per role when its cells and both face sets do
+template <int TX, int TY, int NW>
 constexpr bool tile_fits() {
-    return TX * TY <= NTHREADS && (TX + 1) * TY <= NTHREADS && TX * (TY + 1) <= NTHREADS;
+    return TX * TY <= 64 * NW && (TX + 1) * TY <= 64 * NW && TX * (TY + 1) <= 64 * NW;
 }
 
 struct StageParams {
@@ -252,25 +266,47 @@ __device__ __forceinline__ Views make_views(const StageParams &P) {
     return v;
 }
 
-// Flux through the face between cells c-st and c (byte offsets).  The
-// left/right states are the reference's half-cell extrapolations
-// (HalfSiteExtrapolation.cpp:12-26); emit(n, H_n) receives the 15 components
-// in order.  The nine components the Newton solve needs stay in registers,
-// the other six are reconstructed after it, which keeps the live state small.
-template <int DIR, typename R, bool ROOT_JUMP, typename Guess, typename Load, typename Emit>
-__device__ __forceinline__ void face_flux_from(double t, Guess guess, Load load, Emit emit) {
+// d_i of the pi components entering the axis source of direction DIR
+template <int DIR>
+struct AxisFields {  // pi^{DIR mu} for mu = x, y, eta
+    static constexpr int x = DIR == 1 ? PIXX : DIR == 2 ? PIXY : PIXN;
+    static constexpr int y = DIR == 1 ? PIXY : DIR == 2 ? PIYY : PIYN;
+    static constexpr int n = DIR == 1 ? PIXN : DIR == 2 ? PIYN : PINN;
+};
+
+// Flux through one face.  load(n, j) gives field n at stencil position j
+// (0..3: c-2st .. c+st for the face between cells c-st and c); the left/right
+// states are the reference's half-cell extrapolations
+// (HalfSiteExtrapolation.cpp:12-26); emit(n, H_n) receives the 15 components in
+// order.  start(guess2, v) loads the solves' start |u_T|^2 and, with AX >= 0,
+// the velocity u^DIR / u^tau of the cell whose axis source (SourceTerms.cpp:46-176)
+// is formed on the way: the cell at stencil position AX + 1, whose centred pi
+// differences (times h) are those of positions AX + 2 and AX.  axis(S) receives
+// its four components.  The nine components the recovery needs stay in
+// registers, the other six are loaded and reconstructed after it, which keeps
+// the live state small.
+template <int DIR, typename R, bool ROOT_JUMP, int AX, typename Start, typename Load, typename Emit, typename Axis>
+__device__ __forceinline__ void face_flux(double t, double h, Start start, Load load, Emit emit, Axis axis) {
     constexpr int NN = 9;  // TTT..PITN
-    // all loads of the nine fields first, so that they are in flight together;
-    // load(n, j) gives field n at stencil position j (0..3: c-2st .. c+st)
+    // all loads of the nine fields first, so that they are in flight together
     double raw[NN][4];
 #pragma unroll
     for (int n = 0; n < NN; ++n) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) raw[n][j] = load(n, j);
     }
-    // the Newton guess |u_T|^2 (loads of its own) after the stencil loads, so
-    // that one wait covers both
-    const double guess2 = guess();
+    // the start (loads of its own) after the stencil loads, so that one wait
+    // covers both
+    double guess2, v = 0.0;
+    start(guess2, v);
+    AxisPi<R> ax;
+    if constexpr (AX >= 0) {
+        auto d = [&](int n) { return (R)((raw[n][AX + 2] - raw[n][AX]) * h); };
+        ax.dtt = d(PITT);
+        ax.dtx = d(PITX);
+        ax.dty = d(PITY);
+        ax.dtn = d(PITN);
+    }
     R qL[NN], qR[NN];
 #pragma unroll
     for (int n = 0; n < NN; ++n) {
@@ -298,18 +334,15 @@ __device__ __forceinline__ void face_flux_from(double t, Guess guess, Load load,
         face_values(q0, q1, q2, q3, l, r);
         emit(n, cR * r + cL * l);
     }
-}
-
-// Flux through the face between cells c-st and c (byte offsets).  The
-// left/right states are the reference's half-cell extrapolations
-// (HalfSiteExtrapolation.cpp:12-26); emit(n, H_n) receives the 15 components
-// in order.  The nine components the Newton solve needs stay in registers,
-// the other six are loaded and reconstructed after it.
-template <int DIR, typename R, bool ROOT_JUMP, typename Guess, typename Emit>
-__device__ __forceinline__ void face_flux(double t, Guess guess, const Buf &q, uint32_t f8, uint32_t c,
-                                          uint32_t stp, Emit emit) {
-    face_flux_from<DIR, R, ROOT_JUMP>(
-        t, guess, [&](int n, int j) { return ld(q, c + (uint32_t)j * stp - 2u * stp, n * f8); }, emit);
+    if constexpr (AX >= 0) {
+        auto d = [&](int n) { return (R)((rest[n - NN][AX + 2] - rest[n - NN][AX]) * h); };
+        ax.dix = d(AxisFields<DIR>::x);
+        ax.diy = d(AxisFields<DIR>::y);
+        ax.din = d(AxisFields<DIR>::n);
+        R Sa[4];
+        axis_source<DIR>(ax, (R)v, Sa);
+        axis(Sa);
+    }
 }
 
 // |u_T|^2 at a cell
@@ -318,13 +351,11 @@ __device__ __forceinline__ double uT2_of(const Buf &u, uint32_t f8, uint32_t c) 
     return ux * ux + uy * uy;
 }
 
-// d_i of the pi components entering the axis source of direction DIR
-// (all fourteen loads issued before the differences are formed)
+// d_i of the pi components entering the axis source of direction DIR, from
+// memory (all fourteen loads issued before the differences are formed)
 template <int DIR, typename R>
 __device__ __forceinline__ AxisPi<R> axis_pi(const Buf &q, uint32_t f8, uint32_t s, uint32_t stp, double h) {
-    // pi^{tau mu} (4), then pi^{DIR mu} for mu = x, y, eta
-    constexpr int F[7] = {PITT, PITX, PITY, PITN, DIR == 1 ? PIXX : DIR == 2 ? PIXY : PIXN,
-                          DIR == 1 ? PIXY : DIR == 2 ? PIYY : PIYN, DIR == 1 ? PIXN : DIR == 2 ? PIYN : PINN};
+    constexpr int F[7] = {PITT, PITX, PITY, PITN, AxisFields<DIR>::x, AxisFields<DIR>::y, AxisFields<DIR>::n};
     double up[7], dn[7];
 #pragma unroll
     for (int i = 0; i < 7; ++i) {
@@ -346,12 +377,11 @@ __device__ __forceinline__ AxisPi<R> axis_pi(const Buf &q, uint32_t f8, uint32_t
 
 // one component of the reference's per-direction update:
 // acc += dt * [ (H- - H+)/d  (+ S_axis for the four T^{tau mu} components) ]
-// (the difference in R, the accumulation in double)
-template <typename R>
-__device__ __forceinline__ void add_component(double &acc, int n, R Hm, R Hp, const R (&Sa)[4], R inv_d, double dt) {
-    R r = (Hm - Hp) * inv_d;
+__device__ __forceinline__ void add_component(double &acc, int n, double Hm, double Hp, const double (&Sa)[4],
+                                              double inv_d, double dt) {
+    double r = (Hm - Hp) * inv_d;
     if (n < 4) r += Sa[n];
-    acc += (double)r * dt;
+    acc += r * dt;
 }
 
 // the flux part of one component: acc += dt * (H- - H+)/d, the axis sources
@@ -364,52 +394,6 @@ __device__ __forceinline__ void add_flux(double &acc, double Hm, double Hp, doub
 }
 __device__ __forceinline__ void add_flux(double &acc, float Hm, float Hp, float inv_d, double /*dt_d*/, double dt) {
     acc += (double)((Hm - Hp) * inv_d) * dt;
-}
-
-// acc^{tau mu} += dt * S_axis of every direction, after the source terms.  The
-// loads of all directions (fourteen each) are issued together, one wait for
-// all; the velocities u^i come from the source terms' own loads.
-template <bool D3, typename R>
-__device__ __forceinline__ void add_axis_sources(const StageParams &P, const Views &V, uint32_t s, const SrcIn &in,
-                                                 double iut, double (&acc)[NQ]) {
-    const uint32_t f8 = V.f8;
-    auto fields = [](int dir, int i) {
-        constexpr int T[4] = {PITT, PITX, PITY, PITN};
-        constexpr int X[3] = {PIXX, PIXY, PIXN}, Y[3] = {PIXY, PIYY, PIYN}, Z[3] = {PIXN, PIYN, PINN};
-        return i < 4 ? T[i] : dir == 1 ? X[i - 4] : dir == 2 ? Y[i - 4] : Z[i - 4];
-    };
-    constexpr int ND = D3 ? 3 : 2;
-    const uint32_t stp[3] = {8u, V.sy8, V.sz8};
-    double up[ND][7], dn[ND][7];
-#pragma unroll
-    for (int d = 0; d < ND; ++d) {
-#pragma unroll
-        for (int i = 0; i < 7; ++i) {
-            up[d][i] = ld(V.qin, s + stp[d], fields(d + 1, i) * f8);
-            dn[d][i] = ld(V.qin, s - stp[d], fields(d + 1, i) * f8);
-        }
-    }
-    __builtin_amdgcn_sched_barrier(0);  // keep the loads together (not sunk to their uses)
-    const double h[3] = {P.hx, P.hy, P.hz};
-    const double v[3] = {in.ux * iut, in.uy * iut, in.un * iut};
-#pragma unroll
-    for (int d = 0; d < ND; ++d) {
-        auto dd = [&](int i) { return (R)((up[d][i] - dn[d][i]) * h[d]); };
-        AxisPi<R> a;
-        a.dtt = dd(0);
-        a.dtx = dd(1);
-        a.dty = dd(2);
-        a.dtn = dd(3);
-        a.dix = dd(4);
-        a.diy = dd(5);
-        a.din = dd(6);
-        R Sa[4];
-        if (d == 0) axis_source<1>(a, (R)v[0], Sa);
-        else if (d == 1) axis_source<2>(a, (R)v[1], Sa);
-        else axis_source<3>(a, (R)v[2], Sa);
-#pragma unroll
-        for (int n = 0; n < 4; ++n) acc[n] += (double)Sa[n] * P.dt;
-    }
 }
 
 template <bool D3>
@@ -532,207 +516,294 @@ __device__ __forceinline__ void count_flags(const StageParams &P, bool nan, bool
     }
 }
 
-// One tile of one stage.  Hs holds the x / y face fluxes of the tile
-// (SHARED) or this lane's forward face (reference split); Hz is the eta face
-// carried from the plane below, one slot per lane that only its own lane
-// touches.  R is the arithmetic type of the stencil, fluxes and sources; the
-// tile is TX x TY cells (P.tiles_x / P.tiles_y must be counted with them).
-template <bool D3, bool STAGE2, bool SHARED, typename R, int TX = kTileX, int TY = kTileY>
-__device__ __forceinline__ void stage_tile(const StageParams &P, int tile, R (*Hs)[NTHREADS], R (*Hz)[NTHREADS],
-                                           R *zring) {
-    // split precision in 3+1D: the eta-face stencil of this lane's column is
-    // kept in LDS for three planes (lane-private slots), so each plane's 15
-    // fields are read from memory once by the eta faces instead of four times
-    constexpr bool ZRING = D3 && SHARED && sizeof(R) == 4;
-    auto zr = [&](int plane, int n) -> R & {  // ring slot of a plane (planes >= -1) and field
-        return zring[(((plane + 3) % 3) * NQ + n) * NTHREADS + (int)threadIdx.x];
-    };
-    static_assert(tile_fits<TX, TY>(), "tile does not fit one workgroup");
+// The LDS of a stage workgroup: what the face waves hand to the cell waves for
+// one plane.  Hx / Hy: fluxes through the tile's x / y faces, slot = the face's
+// lane; Dz: difference of the fluxes through a cell's lower and upper eta face;
+// Ax: the axis sources of the three directions.
+template <bool D3, typename R, int NW>
+struct StageLds {
+    static constexpr int NL = 64 * NW;  // lanes per role
+    R Hx[NQ][NL];
+    R Hy[NQ][NL];
+    R Dz[D3 ? NQ : 1][D3 ? NL : 1];
+    R Ax[D3 ? 3 : 2][4][NL];
+};
+
+// a direction as a type
+template <int N>
+struct Dir {
+    static constexpr int value = N;
+};
+
+// a workgroup's part of the lattice
+struct Tile {
+    int i0, j0, k0, k1;
+};
+
+template <int TX, int TY>
+__device__ __forceinline__ Tile tile_at(const StageParams &P, int tile) {
     const int tpl = P.tiles_x * P.tiles_y;
     const int zc = tile / tpl;
     const int txy = tile - zc * tpl;
     const int ty = txy / P.tiles_x;
-    const int tx = txy - ty * P.tiles_x;
-    const int i0 = tx * TX, j0 = ty * TY;
-    const int k0 = zc * P.kz;
-    const int k1 = min(k0 + P.kz, P.nz);
+    Tile T;
+    T.i0 = (txy - ty * P.tiles_x) * TX;
+    T.j0 = ty * TY;
+    T.k0 = zc * P.kz;
+    T.k1 = min(T.k0 + P.kz, P.nz);
+    return T;
+}
 
-    const Views V = make_views(P);
-    const uint32_t f8 = V.f8, sy8 = V.sy8, sz8 = V.sz8;
-    const int tid = (int)threadIdx.x;
-    const uint32_t sy = (uint32_t)P.sy;
-    const double t = P.t_src, dt = P.dt;
-    const R inv_dx = (R)P.inv_dx, inv_dy = (R)P.inv_dy, inv_dz = (R)P.inv_dz;
+// Byte offset of the cell (i, j) of a plane.  Indices one past either end
+// (ghosts) are fine.
+__device__ __forceinline__ uint32_t cell_offset(const StageParams &P, uint32_t plane, int i, int j) {
+    return (plane + (uint32_t)(j + 2) * (uint32_t)P.sy + (uint32_t)(i + 2)) * 8u;
+}
 
-    // this lane's cell
-    const int ci = tid % TX, cj = tid / TX;
-    const int ii = i0 + ci, jj = j0 + cj;
+// Source terms of a cell: acc = q + dt S (eulerStepKernelSource), and the
+// inputs of its recovery.
+template <bool D3, bool STAGE2, typename R>
+__device__ __forceinline__ void cell_sources(const StageParams &P, const Views &V, uint32_t s, double (&acc)[NQ],
+                                             Recovery &rec, double &iut, bool &nan) {
+    const uint32_t f8 = V.f8;
+    double Q[NQ];
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) Q[n] = ld(V.qin, s, n * f8);
+    SrcIn in;
+    load_src_in<D3>(P, V, s, in);
+    R S[NQ];
+    source_terms<R>(P.eos, in, Q, S, nan);
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) acc[n] = Q[n] + P.dt * (double)S[n];
+    iut = rcp(in.ut);
+    // the cell recovery's inputs come from the same loads: e at the stage's
+    // input level (its fallback base) and |u_T| of the velocity that seeds it,
+    // u_cur in stage 1 and u_prev in stage 2
+    // (FullyDiscreteKurganovTadmorScheme.cpp:761-780)
+    rec.e_prev = in.e;
+    rec.uT_guess = STAGE2 ? sqrt_pos(fabs(in.uxp * in.uxp + in.uyp * in.uyp))
+                          : sqrt_pos(fabs(in.ux * in.ux + in.uy * in.uy));
+}
+
+// The cell waves' part of one tile.  Per plane: sources; wait for the plane's
+// fluxes; add them; hand the LDS back; finish the cell.
+template <bool D3, bool STAGE2, typename R, int TX, int TY, int NW>
+__device__ __forceinline__ void cell_role(const StageParams &P, const Views &V, const Tile &T, const StageLds<D3, R, NW> &lds,
+                                          int lane) {
+    const double dt = P.dt;
+    const int ci = lane % TX, cj = lane / TX;
+    const int ii = T.i0 + ci, jj = T.j0 + cj;
     const bool cell_ok = cj < TY && ii < P.nx && jj < P.ny;
-
-    for (int kk = k0; kk < k1; ++kk) {
-        const uint32_t plane = (uint32_t)plane_of(kk, D3) * (uint32_t)P.sz;
-        const uint32_t s = (plane + (uint32_t)(jj + 2) * sy + (uint32_t)(ii + 2)) * 8u;
+    for (int kk = T.k0; kk < T.k1; ++kk) {
+        const uint32_t s = cell_offset(P, (uint32_t)plane_of(kk, D3) * (uint32_t)P.sz, ii, jj);
         bool nan = false, fallback = false;
         double acc[NQ];
         Recovery rec{0.0, 0.0};
-        double iut = 0.0;
-
-        // ---- sources: acc = q + dt S (eulerStepKernelSource)
         if (cell_ok) {
-            double Q[NQ];
-#pragma unroll
-            for (int n = 0; n < NQ; ++n) Q[n] = ld(V.qin, s, n * f8);
-            SrcIn in;
-            load_src_in<D3>(P, V, s, in);
-            R S[NQ];
-            source_terms<R>(P.eos, in, Q, S, nan);
-#pragma unroll
-            for (int n = 0; n < NQ; ++n) acc[n] = Q[n] + dt * (double)S[n];
-            iut = rcp(in.ut);
-            if (SHARED) add_axis_sources<D3, R>(P, V, s, in, iut, acc);
-            // the cell recovery's inputs come from the same loads: e at the
-            // stage's input level (its fallback base) and |u_T| of the velocity
-            // that seeds it, u_cur in stage 1 and u_prev in stage 2
-            // (FullyDiscreteKurganovTadmorScheme.cpp:761-780)
-            rec.e_prev = in.e;
-            rec.uT_guess = STAGE2 ? sqrt_pos(fabs(in.uxp * in.uxp + in.uyp * in.uyp))
-                                  : sqrt_pos(fabs(in.ux * in.ux + in.uy * in.uy));
+            double iut;
+            cell_sources<D3, STAGE2, R>(P, V, s, acc, rec, iut, nan);
         }
-
-        if (SHARED) {
-            // ---- x faces: (TX+1) x TY, face f between cells (fi-1, fj) and (fi, fj)
-            {
-                const int fi = tid % (TX + 1), fj = tid / (TX + 1);
-                const int gi = i0 + fi, gj = j0 + fj;  // interior index of the right cell
-                if (fj < TY && gi <= P.nx && gj < P.ny) {
-                    const uint32_t c = (plane + (uint32_t)(gj + 2) * sy + (uint32_t)(gi + 2)) * 8u;
-                    face_flux<1, R, true>(t, [&] { return uT2_of(V.ucur, f8, c - 8); }, V.qin, f8, c, 8,
-                                    [&](int n, R h) { Hs[n][tid] = h; });
-                }
-            }
-            __syncthreads();
-            if (cell_ok) {
-                const int fm = cj * (TX + 1) + ci;
+        __syncthreads();  // the plane's fluxes are in LDS
+        if (cell_ok) {
+            const R inv_dx = (R)P.inv_dx, inv_dy = (R)P.inv_dy, inv_dz = (R)P.inv_dz;
+            const int fx = cj * (TX + 1) + ci, fy = cj * TX + ci;  // the cell's lower x and y face
 #pragma unroll
-                for (int n = 0; n < NQ; ++n) add_flux(acc[n], Hs[n][fm], Hs[n][fm + 1], inv_dx, P.dt_dx, dt);
+            for (int n = 0; n < 4; ++n) {
+                acc[n] += (double)lds.Ax[0][n][fx] * dt;
+                acc[n] += (double)lds.Ax[1][n][fy] * dt;
+                if constexpr (D3) acc[n] += (double)lds.Ax[2][n][lane] * dt;
             }
-            __syncthreads();
-            // ---- y faces: TX x (TY+1), face f between cells (fi, fj-1) and (fi, fj)
-            {
-                const int fi = tid % TX, fj = tid / TX;
-                const int gi = i0 + fi, gj = j0 + fj;
-                if (fj <= TY && gi < P.nx && gj <= P.ny) {
-                    const uint32_t c = (plane + (uint32_t)(gj + 2) * sy + (uint32_t)(gi + 2)) * 8u;
-                    face_flux<2, R, true>(t, [&] { return uT2_of(V.ucur, f8, c - sy8); }, V.qin, f8, c, sy8,
-                                    [&](int n, R h) { Hs[n][tid] = h; });
-                }
-            }
-            __syncthreads();
-            if (cell_ok) {
-                const int fm = cj * TX + ci;
 #pragma unroll
-                for (int n = 0; n < NQ; ++n) add_flux(acc[n], Hs[n][fm], Hs[n][fm + TX], inv_dy, P.dt_dy, dt);
-            }
-            __syncthreads();
-            // ---- eta faces: solved by the cell's own lane, the upper one carried to the next plane
-            if (D3 && cell_ok) {
-                if (kk == k0) {
-                    if constexpr (ZRING) {
-                        // lower face: planes k0-1 .. k0+1 into the ring first (fifteen
-                        // loads in flight at a time), plane k0-2 from memory
-#pragma unroll
-                        for (int j = 1; j < 4; ++j) {
-                            double v[NQ];
-#pragma unroll
-                            for (int n = 0; n < NQ; ++n) v[n] = ld(V.qin, s + (uint32_t)j * sz8 - 2u * sz8, n * f8);
-#pragma unroll
-                            for (int n = 0; n < NQ; ++n) zr(kk + j - 2, n) = (R)v[n];
-                        }
-                        face_flux_from<3, R, true>(t, [&] { return uT2_of(V.ucur, f8, s - sz8); },
-                            [&](int n, int j) {
-                                return j == 0 ? ld(V.qin, s - 2u * sz8, n * f8) : (double)zr(kk + j - 2, n);
-                            },
-                            [&](int n, R h) { Hz[n][tid] = h; });
-                    } else {
-                        face_flux<3, R, true>(t, [&] { return uT2_of(V.ucur, f8, s - sz8); }, V.qin, f8, s, sz8,
-                                        [&](int n, R h) { Hz[n][tid] = h; });
-                    }
-                }
-                auto upper = [&](int n, R h) {
-                    add_flux(acc[n], Hz[n][tid], h, inv_dz, P.dt_dz, dt);
-                    Hz[n][tid] = h;
-                };
-                if constexpr (ZRING) {
-                    // upper face: planes kk-1 .. kk+1 from the ring, kk+2 from memory (all 15
-                    // loads issued together); plane kk+2 then takes the slot kk-1 leaves
-                    double fresh[NQ];
-#pragma unroll
-                    for (int n = 0; n < NQ; ++n) fresh[n] = ld(V.qin, s + 2u * sz8, n * f8);
-                    face_flux_from<3, R, true>(t, [&] { return uT2_of(V.ucur, f8, s); },
-                        [&](int n, int j) { return j < 3 ? (double)zr(kk - 1 + j, n) : fresh[n]; }, upper);
-#pragma unroll
-                    for (int n = 0; n < NQ; ++n) zr(kk + 2, n) = (R)fresh[n];
-                } else {
-                    face_flux<3, R, true>(t, [&] { return uT2_of(V.ucur, f8, s); }, V.qin, f8, s + sz8, sz8, upper);
-                }
-            }
-        } else if (cell_ok) {
-            // reference work split: both faces of each direction, Newton guess from this cell
-            const double uTs = uT2_of(V.ucur, f8, s);
-            {
-                R Sa[4];
-                axis_source<1>(axis_pi<1, R>(V.qin, f8, s, 8, P.hx), (R)(ld(V.ucur, s, f8) * iut), Sa);
-                face_flux<1, R, false>(t, [&] { return uTs; }, V.qin, f8, s + 8, 8, [&](int n, R h) { Hs[n][tid] = h; });
-                face_flux<1, R, false>(t, [&] { return uTs; }, V.qin, f8, s, 8,
-                                [&](int n, R h) { add_component(acc[n], n, h, Hs[n][tid], Sa, inv_dx, dt); });
-            }
-            {
-                R Sa[4];
-                axis_source<2>(axis_pi<2, R>(V.qin, f8, s, sy8, P.hy), (R)(ld(V.ucur, s, 2 * f8) * iut), Sa);
-                face_flux<2, R, false>(t, [&] { return uTs; }, V.qin, f8, s + sy8, sy8, [&](int n, R h) { Hs[n][tid] = h; });
-                face_flux<2, R, false>(t, [&] { return uTs; }, V.qin, f8, s, sy8,
-                                [&](int n, R h) { add_component(acc[n], n, h, Hs[n][tid], Sa, inv_dy, dt); });
-            }
-            if (D3) {
-                R Sa[4];
-                axis_source<3>(axis_pi<3, R>(V.qin, f8, s, sz8, P.hz), (R)(ld(V.ucur, s, 3 * f8) * iut), Sa);
-                face_flux<3, R, false>(t, [&] { return uTs; }, V.qin, f8, s + sz8, sz8, [&](int n, R h) { Hs[n][tid] = h; });
-                face_flux<3, R, false>(t, [&] { return uTs; }, V.qin, f8, s, sz8,
-                                [&](int n, R h) { add_component(acc[n], n, h, Hs[n][tid], Sa, inv_dz, dt); });
+            for (int n = 0; n < NQ; ++n) {
+                add_flux(acc[n], lds.Hx[n][fx], lds.Hx[n][fx + 1], inv_dx, P.dt_dx, dt);
+                add_flux(acc[n], lds.Hy[n][fy], lds.Hy[n][fy + TX], inv_dy, P.dt_dy, dt);
+                if constexpr (D3) add_flux(acc[n], lds.Dz[n][lane], R(0), inv_dz, P.dt_dz, dt);
             }
         }
-
+        __syncthreads();  // the face waves may write the next plane
         double e_new = 0.0;
         if (cell_ok) e_new = finish_cell<D3, STAGE2>(P, V, s, ii, jj, kk, acc, rec, nan, fallback);
         count_flags(P, nan, fallback, e_new);
     }
 }
 
-// The LDS of a stage workgroup, sized by the template arguments.
-template <bool D3, bool SHARED, typename R>
-struct StageLds {
-    static constexpr bool kRing = D3 && SHARED && sizeof(R) == 4;
-    R Hs[NQ][NTHREADS];
-    R Hz[D3 && SHARED ? NQ : 1][NTHREADS];
-    R Zr[kRing ? 3 : 1][kRing ? NQ : 1][NTHREADS];
-};
+// The face waves' part of one tile.  Per plane: the x faces ((TX+1) x TY, face
+// f between cells f-1 and f), the y faces (TX x (TY+1)) and each cell's upper
+// eta face; the lower one is carried from the plane below.  In 3+1D a lane
+// keeps its column's planes k-1, k, k+1 in registers (90 of the 256; the two
+// x / y solves need about 150), so that an eta face loads one new plane
+// instead of four and the y face takes its own cell from there: 201x201x101
+// 2.68 -> 2.40 ms per step, and the L1 sends a third fewer requests to L2.
+template <bool D3, typename R, int TX, int TY, int NW>
+__device__ __forceinline__ void face_role(const StageParams &P, const Views &V, const Tile &T, StageLds<D3, R, NW> &lds,
+                                          int lane) {
+    const uint32_t f8 = V.f8, sy8 = V.sy8, sz8 = V.sz8;
+    const double t = P.t_src;
+    const int ci = lane % TX, cj = lane / TX;              // y face and cell
+    const int xi = lane % (TX + 1), xj = lane / (TX + 1);  // x face
+    const bool x_ok = xj < TY && T.i0 + xi <= P.nx && T.j0 + xj < P.ny;
+    const bool y_ok = cj <= TY && T.i0 + ci < P.nx && T.j0 + cj <= P.ny;
+    const bool z_ok = D3 && cj < TY && T.i0 + ci < P.nx && T.j0 + cj < P.ny;
+    // a face's start: |u_T|^2 at byte offset g, u^dir / u^tau at c
+    auto start = [&](uint32_t g, uint32_t c, int dir) {
+        return [&V, f8, g, c, dir](double &guess2, double &v) {
+            const double ux = ld(V.ucur, g, f8), uy = ld(V.ucur, g, 2 * f8);
+            const double ut = ld(V.ucur, c, 0), ui = ld(V.ucur, c, dir * f8);
+            guess2 = ux * ux + uy * uy;
+            v = ui * rcp(ut);
+        };
+    };
+    auto axis_to = [&](int d) {
+        return [&lds, d, lane](const R (&S)[4]) {
+#pragma unroll
+            for (int n = 0; n < 4; ++n) lds.Ax[d][n][lane] = S[n];
+        };
+    };
+    R carry[NQ];                                              // flux through the lower eta face
+    double below[D3 ? NQ : 1], here[D3 ? NQ : 1], above[D3 ? NQ : 1];  // planes k-1, k, k+1 of this column
+    if constexpr (D3) {
+        if (z_ok) {
+            const uint32_t s = cell_offset(P, (uint32_t)plane_of(T.k0, D3) * (uint32_t)P.sz, T.i0 + ci, T.j0 + cj);
+            double far[NQ];
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) far[n] = ld(V.qin, s - 2u * sz8, n * f8);
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) below[n] = ld(V.qin, s - sz8, n * f8);
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) here[n] = ld(V.qin, s, n * f8);
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) above[n] = ld(V.qin, s + sz8, n * f8);
+            face_flux<3, R, true, -1>(
+                t, 0.0, [&](double &guess2, double &) { guess2 = uT2_of(V.ucur, f8, s - sz8); },
+                [&](int n, int j) { return j == 0 ? far[n] : j == 1 ? below[n] : j == 2 ? here[n] : above[n]; },
+                [&](int n, R h) { carry[n] = h; }, [](const R (&)[4]) {});
+        }
+    }
+    for (int kk = T.k0; kk < T.k1; ++kk) {
+        const uint32_t plane = (uint32_t)plane_of(kk, D3) * (uint32_t)P.sz;
+        if (x_ok) {
+            const uint32_t c = cell_offset(P, plane, T.i0 + xi, T.j0 + xj);
+            face_flux<1, R, true, 1>(
+                t, P.hx, start(c - 8, c, 1), [&](int n, int j) { return ld(V.qin, c + (uint32_t)j * 8u - 16u, n * f8); },
+                [&](int n, R h) { lds.Hx[n][lane] = h; }, axis_to(0));
+        }
+        const uint32_t s = cell_offset(P, plane, T.i0 + ci, T.j0 + cj);
+        if (y_ok) {
+            face_flux<2, R, true, 1>(
+                t, P.hy, start(s - sy8, s, 2),
+                [&](int n, int j) { return ld(V.qin, s + (uint32_t)j * sy8 - 2u * sy8, n * f8); },
+                [&](int n, R h) { lds.Hy[n][lane] = h; }, axis_to(1));
+        }
+        if constexpr (D3) {
+            if (z_ok) {
+                double fresh[NQ];
+#pragma unroll
+                for (int n = 0; n < NQ; ++n) fresh[n] = ld(V.qin, s + 2u * sz8, n * f8);
+                face_flux<3, R, true, 0>(
+                    t, P.hz, start(s, s, 3),
+                    [&](int n, int j) { return j == 0 ? below[n] : j == 1 ? here[n] : j == 2 ? above[n] : fresh[n]; },
+                    [&](int n, R h) {
+                        lds.Dz[n][lane] = carry[n] - h;
+                        carry[n] = h;
+                    },
+                    axis_to(2));
+#pragma unroll
+                for (int n = 0; n < NQ; ++n) {
+                    below[n] = here[n];
+                    here[n] = above[n];
+                    above[n] = fresh[n];
+                }
+            }
+        }
+        __syncthreads();  // the plane's fluxes are in LDS
+        __syncthreads();  // and have been read
+    }
+}
+
+// One tile of one stage by a workgroup of 2 x 64 NW lanes: the first half are
+// the cell waves, the second the face waves (the split is uniform over each
+// wave).  Both run the same number of barriers, two per plane, and the last one
+// leaves the LDS free for another tile.
+template <bool D3, bool STAGE2, typename R, int TX, int TY, int NW>
+__device__ __forceinline__ void stage_tile(const StageParams &P, int tile, StageLds<D3, R, NW> &lds) {
+    static_assert(tile_fits<TX, TY, NW>(), "tile does not fit its waves");
+    const Views V = make_views(P);
+    const Tile T = tile_at<TX, TY>(P, tile);
+    const int role = __builtin_amdgcn_readfirstlane((int)threadIdx.x / (64 * NW));
+    const int lane = (int)threadIdx.x - role * 64 * NW;
+    if (role != 0)
+        face_role<D3, R, TX, TY, NW>(P, V, T, lds, lane);
+    else
+        cell_role<D3, STAGE2, R, TX, TY, NW>(P, V, T, lds, lane);
+}
+
+// The parameters are read where they are used, through the kernel-argument
+// segment (the kernel's first and only argument, at offset 0), instead of from
+// the argument copy the compiler otherwise keeps in scalar registers across
+// the plane loop: some ninety uniform values there made it spill about three
+// times as many scalar registers and twice as many vector registers as it does
+// reading them in place.
+__device__ __forceinline__ const StageParams &kernarg_params() {
+    typedef __attribute__((address_space(4))) const StageParams KernargParams;
+    return *(const StageParams *)(KernargParams *)__builtin_amdgcn_kernarg_segment_ptr();
+}
 
 // One event: workgroup -> tile (XCD-aware) -> stage_tile.
-template <bool D3, bool STAGE2, bool SHARED, typename R>
-__global__ __launch_bounds__(NTHREADS, D3 ? VAH_BLOCKS_3D : VAH_BLOCKS_2D) void stage_kernel(StageParams P_arg) {
-    // The parameters are read where they are used, through the kernel-argument
-    // segment (P_arg is its first and only argument, at offset 0), instead of
-    // from the argument copy the compiler otherwise keeps in scalar registers
-    // across the plane loop: some ninety uniform values there made it spill
-    // about three times as many scalar registers and twice as many vector
-    // registers as it does reading them in place.
-    typedef __attribute__((address_space(4))) const StageParams KernargParams;
-    const StageParams &P = *(const StageParams *)(KernargParams *)__builtin_amdgcn_kernarg_segment_ptr();
+template <bool D3, bool STAGE2, typename R>
+__global__ __launch_bounds__(128 * kTileWaves, kWavesPerSimd) void stage_kernel(StageParams P_arg) {
+    const StageParams &P = kernarg_params();
     (void)P_arg;
-    __shared__ StageLds<D3, SHARED, R> lds;
+    __shared__ StageLds<D3, R, kTileWaves> lds;
     const int tile = tile_of_block(P, (int)blockIdx.x);
     if (tile < 0) return;  // padding workgroups: no barrier reached
-    stage_tile<D3, STAGE2, SHARED, R>(P, tile, lds.Hs, lds.Hz, &lds.Zr[0][0][0]);
+    stage_tile<D3, STAGE2, R, kTileX, kTileY, kTileWaves>(P, tile, lds);
+}
+
+// The reference's work split (VAH_FLUX_PER_CELL): a lane per cell solves both of
+// its faces in each direction with the cell's own Newton guess.
+template <bool D3, bool STAGE2>
+__global__ __launch_bounds__(kCellThreads, kWavesPerSimd) void stage_per_cell_kernel(StageParams P_arg) {
+    const StageParams &P = kernarg_params();
+    (void)P_arg;
+    __shared__ double Hs[NQ][kCellThreads];  // the lane's forward face
+    const int tile = tile_of_block(P, (int)blockIdx.x);
+    if (tile < 0) return;
+    const Views V = make_views(P);
+    const Tile T = tile_at<kCellTileX, kCellTileY>(P, tile);
+    const uint32_t f8 = V.f8;
+    const double t = P.t_src, dt = P.dt;
+    const int tid = (int)threadIdx.x;
+    const int ii = T.i0 + tid % kCellTileX, jj = T.j0 + tid / kCellTileX;
+    const bool cell_ok = ii < P.nx && jj < P.ny;
+    for (int kk = T.k0; kk < T.k1; ++kk) {
+        const uint32_t s = cell_offset(P, (uint32_t)plane_of(kk, D3) * (uint32_t)P.sz, ii, jj);
+        bool nan = false, fallback = false;
+        double e_new = 0.0;
+        if (cell_ok) {
+            double acc[NQ], iut;
+            Recovery rec{0.0, 0.0};
+            cell_sources<D3, STAGE2, double>(P, V, s, acc, rec, iut, nan);
+            const double uTs = uT2_of(V.ucur, f8, s);
+            auto direction = [&](auto dir, uint32_t stp, double h, double inv_d) {
+                constexpr int DIR = decltype(dir)::value;
+                double Sa[4];
+                axis_source<DIR>(axis_pi<DIR, double>(V.qin, f8, s, stp, h), ld(V.ucur, s, DIR * f8) * iut, Sa);
+                auto face = [&](uint32_t c, auto emit) {
+                    face_flux<DIR, double, false, -1>(
+                        t, 0.0, [&](double &guess2, double &) { guess2 = uTs; },
+                        [&](int n, int j) { return ld(V.qin, c + (uint32_t)j * stp - 2u * stp, n * f8); }, emit,
+                        [](const double (&)[4]) {});
+                };
+                face(s + stp, [&](int n, double H) { Hs[n][tid] = H; });
+                face(s, [&](int n, double H) { add_component(acc[n], n, H, Hs[n][tid], Sa, inv_d, dt); });
+            };
+            direction(Dir<1>{}, 8u, P.hx, P.inv_dx);
+            direction(Dir<2>{}, V.sy8, P.hy, P.inv_dy);
+            if constexpr (D3) direction(Dir<3>{}, V.sz8, P.hz, P.inv_dz);
+            e_new = finish_cell<D3, STAGE2>(P, V, s, ii, jj, kk, acc, rec, nan, fallback);
+        }
+        count_flags(P, nan, fallback, e_new);
+    }
 }
 
 // Zero-gradient ghost copies of an initial state: every face ghost (one index

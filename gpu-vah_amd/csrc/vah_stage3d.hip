@@ -12,19 +12,19 @@ namespace vah {
 
 namespace {
 
-template <bool S2, bool SH, typename R>
+template <bool S2, typename R>
 void launch3(const StageLaunch &L, const StageParams &P) {
-    hipLaunchKernelGGL((stage_kernel<true, S2, SH, R>), dim3(L.grid), dim3(NTHREADS), 0, L.stream, P);
+    hipLaunchKernelGGL((stage_kernel<true, S2, R>), dim3(L.grid), dim3(128 * kTileWaves), 0, L.stream, P);
 }
 
 template <bool S2>
 void variant3(const StageLaunch &L, const StageParams &P) {
     if (L.precision == VAH_FP32_SPLIT)
-        launch3<S2, true, float>(L, P);
+        launch3<S2, float>(L, P);
     else if (L.flux_mode == VAH_FLUX_SHARED)
-        launch3<S2, true, double>(L, P);
+        launch3<S2, double>(L, P);
     else
-        launch3<S2, false, double>(L, P);
+        hipLaunchKernelGGL((stage_per_cell_kernel<true, S2>), dim3(L.grid), dim3(kCellThreads), 0, L.stream, P);
 }
 
 }  // namespace

@@ -81,7 +81,7 @@ typedef struct vah_batch_status {
 
 typedef struct vah_batch_variant {
     int tile_x, tile_y;        /* cells per workgroup tile */
-    int blocks_per_cu;         /* workgroups per CU the registers are sized for */
+    int blocks_per_cu;         /* waves per SIMD the registers are sized for */
     int kz;                    /* eta planes per 3+1D tile */
 } vah_batch_variant;
 
