@@ -19,6 +19,7 @@
 #include <stdint.h>
 
 #include "vah_eos_wb.h"
+#include "vah_face.h"
 #include "vah_log.h"
 #include "vah_sqrt.h"
 #include "vah_tanh.h"
@@ -130,41 +131,63 @@ __device__ __forceinline__ double conformal_T(double e, const uint32_t *__restri
     return (double)T;
 }
 
-__device__ __forceinline__ void table_lookup(const Eos &E, double e, double *p, double *T) {
-    double f = (eos_log(e) - E.lne0) * E.inv_h;
-    int last = E.n - 1;
-    if (!(f >= 0.0)) {
-        double r = e / E.e_first;
-        if (p) *p = E.p[0] * r;
-        if (T) *T = E.T[0] * __builtin_sqrt(__builtin_sqrt(r));
-        return;
-    }
-    int i = (int)f;
-    if (i >= last) {
-        double r = e / E.e_last;
-        if (p) *p = E.p[last] * r;
-        if (T) *T = E.T[last] * __builtin_sqrt(__builtin_sqrt(r));
-        return;
-    }
-    double w = f - (double)i;
-    if (p) *p = E.p[i] + w * (E.p[i + 1] - E.p[i]);
-    if (T) *T = E.T[i] + w * (E.T[i + 1] - E.T[i]);
+// a - b, a rounded first.  Contracted into the product that gives the node position
+// the weight would differ from the host's in most cells by 1e-13, p by an ulp: the
+// initial p of a single lattice is formed on the host, a batch event's on the device.
+__device__ __forceinline__ double uncontracted_sub(double a, double b) {
+#pragma clang fp contract(off)
+    return a - b;
 }
 
+__device__ __forceinline__ double table_T(const Eos &E, double e) {
+    double f = (eos_log(e) - E.lne0) * E.inv_h;
+    int last = E.n - 1;
+    if (!(f >= 0.0)) return E.T[0] * __builtin_sqrt(__builtin_sqrt(e / E.e_first));
+    int i = (int)f;
+    if (i >= last) return E.T[last] * __builtin_sqrt(__builtin_sqrt(e / E.e_last));
+    double w = uncontracted_sub(f, (double)i);
+    return __builtin_fma(w, E.T[i + 1] - E.T[i], E.T[i]);
+}
+
+// p(e) in two halves, so that the table's load latency overlaps whatever the
+// caller does between them: begin() finds the nodes and issues their loads,
+// end() interpolates (linear in ln e, power laws outside).
+struct EosP {
+    double e, w, p0, p1;
+    int at;  // 0: between nodes; -1, 1: below, above the table
+
+    __device__ __forceinline__ void begin(const Eos &E, double e_) {
+        e = e_;
+        if (E.kind != 1) return;
+        const double f = (eos_log(e) - E.lne0) * E.inv_h;
+        const int last = E.n - 1;
+        const bool below = !(f >= 0.0);
+        const int i = below ? 0 : (int)__builtin_fmin(f, (double)last);
+        at = below ? -1 : i >= last;
+        w = uncontracted_sub(f, (double)i);
+        const int k = i < last ? i : last - 1;
+        p0 = E.p[k];
+        p1 = E.p[k + 1];
+    }
+    __device__ __forceinline__ double end(const Eos &E) const {
+        if (E.kind == 0) return e * kThird;
+        if (E.kind == 2) return wb_pressure(e);
+        double p = __builtin_fma(w, p1 - p0, p0);
+        if (at != 0) p = at < 0 ? p0 * (e / E.e_first) : p1 * (e / E.e_last);
+        return p;
+    }
+};
+
 __device__ __forceinline__ double eos_p(const Eos &E, double e) {
-    if (E.kind == 0) return e * kThird;
-    if (E.kind == 2) return wb_pressure(e);
-    double p;
-    table_lookup(E, e, &p, nullptr);
-    return p;
+    EosP p;
+    p.begin(E, e);
+    return p.end(E);
 }
 
 __device__ __forceinline__ double eos_T(const Eos &E, double e) {
     if (E.kind == 0) return conformal_T(e, E.powf_fix);
     if (E.kind == 2) return wb_temperature(e);
-    double T;
-    table_lookup(E, e, nullptr, &T);
-    return T;
+    return table_T(E, e);
 }
 
 // ---------------------------------------------------------------------------
@@ -350,7 +373,7 @@ __device__ __forceinline__ void face_values(float q0, float q1, float q2, float 
 // Newton recovery of (e, p, u^mu) from T^tau-mu, P_L, pi^tau-mu.
 // ---------------------------------------------------------------------------
 struct Prim {
-    double e, p, ut, ux, uy, un;
+    double e, ut, ux, uy, un;
     int ok;       // 1 converged, 0 fallback
 };
 
@@ -390,13 +413,27 @@ __device__ __forceinline__ bool newton_uT(double t, double uT0, double MB0, doub
 }
 
 // getInferredVariables with W = Pi = 0 (EnergyMomentumTensor.cpp:74-197):
-// then F = A = M3/(M0+P_L), MB = M.
+// then F = A = M3/(M0+P_L), MB = M.  uT2_guess: |u_T|^2 of the velocity that
+// seeds the solve.  In closed form (vah_face.h) wherever the iteration must end
+// on the root, by the iteration in the other lanes.  p is left to the caller.
 template <typename Q>
-__device__ __forceinline__ Prim recover(const Eos &E, double t, const Q &q, double ePrev, double uT_guess) {
+__device__ __forceinline__ Prim recover(double t, const Q &q, double ePrev, double uT2_guess) {
     double M0 = (double)q[TTT] - (double)q[PITT];
     double M1 = (double)q[TTX] - (double)q[PITX];
     double M2 = (double)q[TTY] - (double)q[PITY];
     double M3 = (double)q[TTN] - (double)q[PITN];
+    Prim r;
+    {
+        CellRoot c;
+        const bool ok = cell_root(t, M0, M1, M2, M3, (double)q[PL], face_start(uT2_guess), &c);
+        r.e = c.e;
+        r.ut = c.ut;
+        r.ux = c.ux;
+        r.uy = c.uy;
+        r.un = c.un;
+        r.ok = 1;
+        if (ok) return r;
+    }
     double M0PL = M0 + (double)q[PL];
     if (M0PL == 0.0) M0PL = 1.e-16;
     double F = fdiv(M3, M0PL);
@@ -405,8 +442,7 @@ __device__ __forceinline__ Prim recover(const Eos &E, double t, const Q &q, doub
     double MBT = sqrt_pos(M1 * M1 + M2 * M2);
     if (MBT == 0.0) MBT = 1.e-16;
     double uT = 0.0;
-    Prim r;
-    if (newton_uT(t, uT_guess, M0, MBT, M3, (double)q[PL], Ft, x, uT)) {
+    if (newton_uT(t, sqrt_pos(uT2_guess), M0, MBT, M3, (double)q[PL], Ft, x, uT)) {
         double C2 = 1.0 + uT * uT;
         double iC = rsqrt(C2);
         double C = C2 * iC;
@@ -426,7 +462,6 @@ __device__ __forceinline__ Prim recover(const Eos &E, double t, const Q &q, doub
         r.ut = 1.0;
         r.ok = 0;
     }
-    r.p = eos_p(E, r.e);
     return r;
 }
 

@@ -1,0 +1,35 @@
+// vah_div.h -- quotients from the hardware's reciprocal estimate, about half the
+// instructions of the correctly rounded sequence, whose range scaling the callers'
+// operands do not need.
+#pragma once
+
+namespace vah {
+
+// hardware estimates on the device, the plain quotients on the host
+__host__ __device__ inline double rcp_estimate(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_rcp(x);
+#else
+    return 1.0 / x;
+#endif
+}
+
+__host__ __device__ inline double rsq_estimate(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_rsq(x);
+#else
+    return 1.0 / __builtin_sqrt(x);
+#endif
+}
+
+// a / b: the estimate refined twice, then a residual correction (~1 ulp for
+// normal operands)
+__host__ __device__ inline double quotient(double a, double b) {
+    double r = rcp_estimate(b);
+    r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+    r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+    const double q = a * r;
+    return __builtin_fma(__builtin_fma(-b, q, a), r, q);
+}
+
+}  // namespace vah

@@ -18,6 +18,8 @@
 
 #include <math.h>
 
+#include "vah_div.h"
+
 namespace vah {
 
 // 1/23, 1/21, ..., 1/3: the series coefficients, highest first.  In device
@@ -41,7 +43,7 @@ __host__ __device__ inline double eos_log(double x) {
         m *= 2.0;
         k -= 1;
     }
-    const double s = (m - 1.0) / (m + 1.0);
+    const double s = quotient(m - 1.0, m + 1.0);
     const double z = s * s;
     double p = kEosLogCoef[0];
     for (int j = 1; j < 11; ++j) p = fma(p, z, kEosLogCoef[j]);

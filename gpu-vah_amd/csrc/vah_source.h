@@ -275,28 +275,25 @@ __device__ __forceinline__ void axis_source(const AxisPi<R> &d, R v, R (&S)[4]) 
     S[3] = d.dtn * v - d.din;
 }
 
-// Regulator (FullyDiscreteKurganovTadmorScheme.cpp:540-665), in place.
+// Regulator (FullyDiscreteKurganovTadmorScheme.cpp:540-665), in place.  pe holds
+// the loads of p(e) in flight; p is formed here, after all that does not need it.
 template <typename QA>
-__device__ __forceinline__ void regulate(double t, QA &q, double &e, double &p, double ut, double ux, double uy,
-                                         double un) {
-    if (e < 0.0) {
-        e = 1.e-7;
-        p = 1.e-7;
-    }
+__device__ __forceinline__ void regulate(double t, const Eos &E, const EosP &pe, QA &q, double &e, double &p,
+                                         double ut, double ux, double uy, double un) {
+    const bool floor_e = e < 0.0;
+    if (floor_e) e = 1.e-7;
     if (q[PL] < 0.0) q[PL] = 1.e-7;
     const double pl = q[PL];
-    const double ptHat = pt_hat(e, p, pl);
+    const double rb = rbar0(powers_of(fdiv(pl, e)));
     const double pitt = q[PITT], pitx = q[PITX], pity = q[PITY], pitn = q[PITN], pixx = q[PIXX], pixy = q[PIXY],
                  pixn = q[PIXN], piyy = q[PIYY], piyn = q[PIYN], pinn = q[PINN];
     const double isF = rsqrt(1.0 + ux * ux + uy * uy);
     const double z0 = t * un * isF;
-    const double z3 = ut / t * isF;
+    const double z3 = fdiv(ut, t) * isF;
     const double t2 = t * t;
-    const double sTrsTrs = sqrt_pos(fabs(e * e + pl * pl + 2.0 * ptHat * ptHat));
     const double pipi = pitt * pitt - 2.0 * pitx * pitx - 2.0 * pity * pity + pixx * pixx + 2.0 * pixy * pixy +
                         piyy * piyy - 2.0 * pitn * pitn * t2 + 2.0 * pixn * pixn * t2 + 2.0 * piyn * piyn * t2 +
                         pinn * pinn * t2 * t2;
-    const double spipi = sqrt_pos(fabs(pipi));
     const double ar[9] = {pitt - pixx - piyy - pinn * t2,
                           -pitn * t2 * un + pitt * ut - pitx * ux - pity * uy,
                           -pixn * t2 * un + pitx * ut - pixx * ux - pixy * uy,
@@ -308,13 +305,22 @@ __device__ __forceinline__ void regulate(double t, QA &q, double &e, double &p, 
                           z0 * pitn - t2 * z3 * pinn};
     // ratios to spipi; a zero spipi makes them 0 * inf = NaN (or +-inf for a
     // nonzero numerator), as the quotients would be
-    double rho = spipi / sTrsTrs;
-    const double ispipi = 1.0 / spipi;
-#pragma unroll
-    for (int m = 0; m < 9; ++m) {
-        double am = ar[m] * ispipi;
-        if (am > rho) rho = am;
+    const double pipi2 = fabs(pipi);
+    double ispipi = rsqrt(pipi2), spipi = pipi2 * ispipi;
+    if (!(pipi2 > 1e-280 && pipi2 < 1e280)) {
+        spipi = __builtin_sqrt(pipi2);
+        ispipi = 1.0 / spipi;
     }
+    double am = ar[0] * ispipi;
+#pragma unroll
+    for (int m = 1; m < 9; ++m) am = __builtin_fmax(am, ar[m] * ispipi);
+    p = pe.end(E);
+    if (floor_e) p = 1.e-7;
+    const double ptHat = 0.5 * ((e - pl) - rb * (e - 3.0 * p));
+    const double s2 = fabs(e * e + pl * pl + 2.0 * ptHat * ptHat);
+    double rho = spipi * rsqrt(s2);
+    if (!(s2 > 1e-280 && s2 < 1e280)) rho = spipi / __builtin_sqrt(s2);
+    if (am > rho) rho = am;
     double fac = tanh_over_x(rho);  // tanh(rho) / rho
     if (rho < 1.e-7) fac = 1.0;
 #pragma unroll

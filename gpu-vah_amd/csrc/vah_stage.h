@@ -445,9 +445,9 @@ __device__ __forceinline__ void load_src_in(const StageParams &P, const Views &V
 }
 
 // Inputs of a cell's recovery besides its conserved variables: the e its
-// fallback scales and the |u_T| its Newton solve starts from.
+// fallback scales and the |u_T|^2 its solve starts from.
 struct Recovery {
-    double e_prev, uT_guess;
+    double e_prev, uT2_guess;
 };
 
 // Stage-2 convex combination, recovery, regulation, store with ghost copies.
@@ -463,11 +463,13 @@ __device__ __forceinline__ double finish_cell(const StageParams &P, const Views 
 #pragma unroll
         for (int n = 0; n < NQ; ++n) acc[n] = 0.5 * (acc[n] + qn[n]);
     }
-    Prim r = recover(P.eos, P.t_rec, acc, rec.e_prev, rec.uT_guess);
+    Prim r = recover(P.t_rec, acc, rec.e_prev, rec.uT2_guess);
+    EosP pe;
+    pe.begin(P.eos, r.e);
     nan = nan || prim_nan(r);
     fallback = !r.ok;
-    double e = r.e, p = r.p;
-    regulate(P.t_rec, acc, e, p, r.ut, r.ux, r.uy, r.un);
+    double e = r.e, p;
+    regulate(P.t_rec, P.eos, pe, acc, e, p, r.ut, r.ux, r.uy, r.un);
     double vals[NQ + 6];
 #pragma unroll
     for (int n = 0; n < NQ; ++n) vals[n] = acc[n];
@@ -581,8 +583,7 @@ __device__ __forceinline__ void cell_sources(const StageParams &P, const Views &
     // u_cur in stage 1 and u_prev in stage 2
     // (FullyDiscreteKurganovTadmorScheme.cpp:761-780)
     rec.e_prev = in.e;
-    rec.uT_guess = STAGE2 ? sqrt_pos(fabs(in.uxp * in.uxp + in.uyp * in.uyp))
-                          : sqrt_pos(fabs(in.ux * in.ux + in.uy * in.uy));
+    rec.uT2_guess = STAGE2 ? in.uxp * in.uxp + in.uyp * in.uyp : in.ux * in.ux + in.uy * in.uy;
 }
 
 // The cell waves' part of one tile.  Per plane: sources; wait for the plane's

@@ -15,6 +15,8 @@
 
 #include <math.h>
 
+#include "vah_div.h"
+
 namespace vah {
 
 // 1/13!, 1/12!, ..., 1/2!, highest first
@@ -44,7 +46,7 @@ __host__ __device__ inline double expm1_small(double y) {
 __host__ __device__ inline double tanh_over_x(double x) {
     if (x > 20.0) return 1.0 / x;
     const double E = expm1_small(2.0 * x);
-    return E / ((E + 2.0) * x);
+    return quotient(E, (E + 2.0) * x);
 }
 
 }  // namespace vah
