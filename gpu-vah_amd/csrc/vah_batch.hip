@@ -29,6 +29,7 @@
 #include "vah_batch_kernels.h"
 #include "vah_glauber.h"
 #include "vah_host_common.h"
+#include "vah_transfer.h"
 
 using namespace vah;
 using vah_host::fail;
@@ -118,6 +119,7 @@ struct vah_batch {
     };
     Staging stage[4];
     int stage_next;
+    vah_host::Transfer transfer;  // fields of events to the host
 };
 
 namespace {
@@ -536,6 +538,8 @@ int vah_batch_create(const vah_batch_options *opt_in, vah_batch **out) {
     b->cap2 = b->cap3 = 4096;
     if (hipMalloc(&b->tiles_dev, sizeof(int2) * (b->cap2 + b->cap3)) != hipSuccess)
         return cleanup(fail(VAH_ERR_NOMEM, "vah_batch_create: tile lists"));
+    if (b->transfer.reserve(4 << 20, 0) != hipSuccess)
+        return cleanup(fail(VAH_ERR_NOMEM, "vah_batch_create: transfer slots"));
     std::string err;
     int rc = vah_host::make_device_eos(opt.eos, opt.table, b->stream, &b->eos, &b->powf_fix, &b->eos_dev, &b->heos,
                                        &err);
@@ -828,21 +832,13 @@ int vah_batch_get_state(vah_batch *b, int slot, double *q, double *e, double *p,
     const HostEvent &h = b->events[slot];
     const long long n = d.nstep;
     const int a = (n & 1) ? 2 : 0, uc = (int)(n & 1);
-    std::vector<double> buf;
-    auto get = [&](const double *src, int nf, double *dst) -> int {
-        if (!dst) return VAH_OK;
-        buf.resize((size_t)nf * h.lay.fs);
-        HIP_TRY(hipMemcpyAsync(buf.data(), src, sizeof(double) * nf * h.lay.fs, hipMemcpyDeviceToHost, b->stream));
-        HIP_TRY(hipStreamSynchronize(b->stream));
-        h.lay.unpad(nf, buf.data(), dst);
-        return VAH_OK;
-    };
-    int rc;
-    if ((rc = get(h.dev.q[a], NQ, q)) != VAH_OK) return rc;
-    if ((rc = get(h.dev.e[0], 1, e)) != VAH_OK) return rc;
-    if ((rc = get(h.dev.p[0], 1, p)) != VAH_OK) return rc;
-    if ((rc = get(h.dev.u[uc], 4, u)) != VAH_OK) return rc;
-    if ((rc = get(h.dev.u[1 - uc], 4, up)) != VAH_OK) return rc;
+    std::vector<vah_host::Segment> segs;
+    if (q) segs.push_back({h.dev.q[a], NQ, q, nullptr});
+    if (e) segs.push_back({h.dev.e[0], 1, e, nullptr});
+    if (p) segs.push_back({h.dev.p[0], 1, p, nullptr});
+    if (u) segs.push_back({h.dev.u[uc], 4, u, nullptr});
+    if (up) segs.push_back({h.dev.u[1 - uc], 4, up, nullptr});
+    HIP_TRY(b->transfer.download(b->device, b->stream, vah_host::Rows(h.lay), segs));
     return VAH_OK;
 }
 

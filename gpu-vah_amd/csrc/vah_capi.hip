@@ -25,6 +25,7 @@
 
 #include "../../include/vah.h"
 #include "vah_host_common.h"
+#include "vah_transfer.h"
 #include "vah_stage.h"
 
 using namespace vah;
@@ -159,6 +160,7 @@ struct vah_ctx {
     Eos eos;
     vah_host::HostEos heos;
     vah_host::Layout lay;
+    vah_host::Transfer transfer;
     long long nstep;
     bool have_state;
     bool stepped;          // a step has completed since the last vah_set_state
@@ -354,23 +356,6 @@ int fill_ghosts(vah_ctx *c) {
                        c->qset[c->qi], c->ebuf[c->ecur], c->pbuf[c->ecur], c->useq[c->uc], c->fs, c->lat.nx, c->lat.ny,
                        c->lat.nz, (long)c->ncx, (long)c->ncx * c->ncy, c->lat.nz > 1 ? 1 : 0, nullptr);
     HIP_TRY(hipGetLastError());
-    return VAH_OK;
-}
-
-// copy interior host arrays into the padded device layout of one slab
-int upload_fields(vah_ctx *c, double *dst_slab, int nfields, const double *src, std::vector<double> &stage_buf) {
-    c->lay.pad(nfields, src, stage_buf);
-    HIP_TRY(hipMemcpyAsync(dst_slab, stage_buf.data(), sizeof(double) * nfields * c->fs, hipMemcpyHostToDevice,
-                           c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return VAH_OK;
-}
-
-int download_fields(vah_ctx *c, const double *src_slab, int nfields, double *dst) {
-    std::vector<double> buf((size_t)nfields * c->fs);
-    HIP_TRY(hipMemcpyAsync(buf.data(), src_slab, sizeof(double) * nfields * c->fs, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    c->lay.unpad(nfields, buf.data(), dst);
     return VAH_OK;
 }
 
@@ -745,6 +730,8 @@ int vah_create(const vah_lattice *lat, const vah_hydro *hydro, const vah_options
         c->nblocks = g.nblocks;
         c->grid = g.grid;
     }
+    if (c->transfer.reserve(sizeof(double) * 25 * c->fs, sizeof(double) * (c->ncx + 64)) != hipSuccess)
+        return cleanup(fail(VAH_ERR_NOMEM, "vah_create: transfer slots"));
     c->red_blocks = 1024;
     if (hipMalloc(&c->red_buf, sizeof(double) * 4 * c->red_blocks) != hipSuccess)
         return cleanup(fail(VAH_ERR_NOMEM, "vah_create: reduction buffer"));
@@ -784,13 +771,13 @@ int vah_set_state(vah_ctx *c, long long nstep, const double *q, const double *e,
     if (!c || !q || !e || !p || !u || !up) return fail(VAH_ERR_ARG, "vah_set_state: NULL argument");
     if (nstep < 0) return fail(VAH_ERR_ARG, "vah_set_state: negative step count");
     HIP_TRY(hipSetDevice(c->device));
-    std::vector<double> buf;
+    HIP_TRY(c->transfer.upload(c->device, c->stream, vah_host::Rows(c->lay),
+                               {{c->qset[c->qi], NQ, nullptr, q},
+                                {c->ebuf[c->ecur], 1, nullptr, e},
+                                {c->pbuf[c->ecur], 1, nullptr, p},
+                                {c->useq[c->uc], 4, nullptr, u},
+                                {c->useq[c->up], 4, nullptr, up}}));
     int rc;
-    if ((rc = upload_fields(c, c->qset[c->qi], NQ, q, buf)) != VAH_OK) return rc;
-    if ((rc = upload_fields(c, c->ebuf[c->ecur], 1, e, buf)) != VAH_OK) return rc;
-    if ((rc = upload_fields(c, c->pbuf[c->ecur], 1, p, buf)) != VAH_OK) return rc;
-    if ((rc = upload_fields(c, c->useq[c->uc], 4, u, buf)) != VAH_OK) return rc;
-    if ((rc = upload_fields(c, c->useq[c->up], 4, up, buf)) != VAH_OK) return rc;
     if ((rc = fill_ghosts(c)) != VAH_OK) return rc;
     // NaN and fallback counts restart with the new state
     HIP_TRY(hipMemsetAsync(c->counters, 0, 4 * sizeof(unsigned), c->stream));
@@ -857,12 +844,13 @@ int vah_synchronize(vah_ctx *c) {
 int vah_get_state(vah_ctx *c, double *q, double *e, double *p, double *u, double *up) {
     if (!c) return fail(VAH_ERR_ARG, "vah_get_state: NULL context");
     HIP_TRY(hipSetDevice(c->device));
-    int rc;
-    if (q && (rc = download_fields(c, c->qset[c->qi], NQ, q)) != VAH_OK) return rc;
-    if (e && (rc = download_fields(c, c->ebuf[c->ecur], 1, e)) != VAH_OK) return rc;
-    if (p && (rc = download_fields(c, c->pbuf[c->ecur], 1, p)) != VAH_OK) return rc;
-    if (u && (rc = download_fields(c, c->useq[c->uc], 4, u)) != VAH_OK) return rc;
-    if (up && (rc = download_fields(c, c->useq[c->up], 4, up)) != VAH_OK) return rc;
+    std::vector<vah_host::Segment> segs;
+    if (q) segs.push_back({c->qset[c->qi], NQ, q, nullptr});
+    if (e) segs.push_back({c->ebuf[c->ecur], 1, e, nullptr});
+    if (p) segs.push_back({c->pbuf[c->ecur], 1, p, nullptr});
+    if (u) segs.push_back({c->useq[c->uc], 4, u, nullptr});
+    if (up) segs.push_back({c->useq[c->up], 4, up, nullptr});
+    HIP_TRY(c->transfer.download(c->device, c->stream, vah_host::Rows(c->lay), segs));
     return VAH_OK;
 }
 
@@ -919,9 +907,10 @@ int vah_validity(vah_ctx *c, double *kn_T, double *kn_L, double *kn, double *r_p
                        1 / c->lat.dx / 2, 1 / c->lat.dy / 2, 1 / c->lat.dz / 2, c->eos, out);
     HIP_TRY(hipGetLastError());
     double *dst[5] = {kn_T, kn_L, kn, r_pi, r_pi2};
+    std::vector<vah_host::Segment> segs;
     for (int f = 0; f < 5; ++f)
-        if (dst[f])
-            HIP_TRY(hipMemcpyAsync(dst[f], out + (size_t)f * n, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
+        if (dst[f]) segs.push_back({out + (size_t)f * n, 1, dst[f], nullptr});
+    HIP_TRY(c->transfer.download(c->device, c->stream, vah_host::Rows(c->lat.nx, c->lat.ny, c->lat.nz), segs));
     HIP_TRY(hipStreamSynchronize(c->stream));
     return VAH_OK;
 }

@@ -101,24 +101,6 @@ struct Layout {
         fs = (ncell + 63) / 64 * 64;
     }
     long interior() const { return (long)nx * ny * nz; }
-    long index(long m) const {
-        int i = (int)(m % nx);
-        int j = (int)((m / nx) % ny);
-        int k = (int)(m / ((long)nx * ny));
-        return (long)vah::plane_of(k, nz > 1) * ncx * ncy + (long)(j + 2) * ncx + (i + 2);
-    }
-    // interior field-major host arrays -> padded slab image (ghosts 0)
-    void pad(int nfields, const double *src, std::vector<double> &dst) const {
-        const long n = interior();
-        dst.assign((size_t)nfields * fs, 0.0);
-        for (int f = 0; f < nfields; ++f)
-            for (long m = 0; m < n; ++m) dst[(size_t)f * fs + index(m)] = src[(size_t)f * n + m];
-    }
-    void unpad(int nfields, const double *src, double *dst) const {
-        const long n = interior();
-        for (int f = 0; f < nfields; ++f)
-            for (long m = 0; m < n; ++m) dst[(size_t)f * n + m] = src[(size_t)f * fs + index(m)];
-    }
 };
 
 // Device EOS: uploads the table (or the powf bitmap of the conformal EOS) on

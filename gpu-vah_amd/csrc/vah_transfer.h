@@ -1,0 +1,230 @@
+// vah_transfer.h -- states between the padded device fields and the caller's
+// interior arrays.
+//
+// What bounds a transfer is the host side: e, p and u of 201x201x101 cells (196 MB)
+// were copied whole into a pageable buffer, its pages touched for the first time,
+// then picked out of it cell by cell with two divisions per element, and took 130 of
+// the 226 ms of an output interval of 40 steps (97 ms now).  A checkpoint of 201x201
+// cells (25 fields up, 30 down) went from 6.9 to 1.5 ms.
+// Here chunks of at most kSlotBytes go through pinned slots, whole rows are copied
+// between a slot and the caller's array while the next chunk is on the link, and
+// from kParallelBytes on kWorkers host threads share the chunks (one thread copies
+// rows at about 10 GB/s, a fifth of the link).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <string.h>
+
+#include <algorithm>
+#include <mutex>
+#include <new>
+#include <thread>
+#include <vector>
+
+#include "vah_host_common.h"
+
+namespace vah_host {
+
+// Rows of the device fields: x fastest, g ghost cells on each side in x and y, gz
+// in eta, fields fs elements apart.
+struct Rows {
+    long nx, ny, nz, g, gz, fs;
+    explicit Rows(const Layout &l) : nx(l.nx), ny(l.ny), nz(l.nz), g(2), gz(l.nz > 1 ? 2 : 0), fs(l.fs) {}
+    // interior cells alone, one field after the other
+    Rows(long nx_, long ny_, long nz_) : nx(nx_), ny(ny_), nz(nz_), g(0), gz(0), fs(nx_ * ny_ * nz_) {}
+    long length() const { return nx + 2 * g; }
+    long per_field() const { return (ny + 2 * g) * (nz + 2 * gz); }
+    // first element of row r, counted over all fields; the row after a field's last
+    // starts the next field, so the gap between fields belongs to the last row
+    long start(long r) const { return r / per_field() * fs + r % per_field() * length(); }
+    // index of the row's first interior cell among the caller's elements, -1 for a ghost row
+    long interior(long r) const {
+        const long f = r / per_field(), s = r % per_field(), j = s % (ny + 2 * g) - g, k = s / (ny + 2 * g) - gz;
+        return j < 0 || j >= ny || k < 0 || k >= nz ? -1 : ((f * nz + k) * ny + j) * nx;
+    }
+    // slot image of rows [r0, r1) -> the caller's array, and back (ghosts and gaps 0)
+    void out(long r0, long r1, const double *slot, double *dst) const {
+        for (long r = r0; r < r1; ++r) {
+            const long m = interior(r);
+            if (m >= 0) memcpy(dst + m, slot + (start(r) - start(r0)) + g, sizeof(double) * nx);
+        }
+    }
+    void in(long r0, long r1, const double *src, double *slot) const {
+        for (long r = r0; r < r1; ++r) {
+            const long m = interior(r), at = start(r) - start(r0), end = start(r + 1) - start(r0);
+            double *row = slot + at;
+            if (m < 0) {
+                memset(row, 0, sizeof(double) * (end - at));
+                continue;
+            }
+            memset(row, 0, sizeof(double) * g);
+            memcpy(row + g, src + m, sizeof(double) * nx);
+            memset(row + g + nx, 0, sizeof(double) * (end - at - g - nx));
+        }
+    }
+};
+
+// nf fields at dev, and the caller's array (one of the two by direction).
+struct Segment {
+    double *dev;
+    int nf;
+    double *dst;
+    const double *src;
+};
+
+// Pinned slots of one context or batch.  Transfers on one object from several
+// threads take turns.
+class Transfer {
+  public:
+    ~Transfer() { release(); }
+
+    // Slots for transfers of up to `bytes` in rows of `row` bytes: called when the
+    // owner is created, and again by transfers that need more.
+    hipError_t reserve(size_t bytes, size_t row) {
+        std::lock_guard<std::mutex> hold(lock_);
+        return grow(bytes, row);
+    }
+    hipError_t download(int device, hipStream_t stream, const Rows &R, const std::vector<Segment> &segs) {
+        return guarded(device, stream, R, segs, false);
+    }
+    hipError_t upload(int device, hipStream_t stream, const Rows &R, const std::vector<Segment> &segs) {
+        return guarded(device, stream, R, segs, true);
+    }
+
+  private:
+    static constexpr size_t kSlotBytes = 2 << 20;
+    static constexpr size_t kParallelBytes = 16 << 20;  // below, starting threads costs what they save
+    static constexpr int kWorkers = 4, kDepth = 2;      // slots per worker: one on the link, one being copied
+
+    std::mutex lock_;
+    char *slots_ = nullptr;
+    bool pinned_ = false;
+    int nslots_ = 0;
+    size_t slot_bytes_ = 0;
+    hipEvent_t done_[kWorkers * kDepth] = {};
+
+    void release() {
+        for (hipEvent_t &e : done_)
+            if (e) (void)hipEventDestroy(e);
+        if (pinned_) (void)hipHostFree(slots_);
+        else delete[] slots_;
+        slots_ = nullptr;
+        nslots_ = 0;
+        slot_bytes_ = 0;
+    }
+
+    hipError_t grow(size_t bytes, size_t row) {
+        const int n = kDepth * (bytes >= kParallelBytes ? kWorkers : 1);
+        const size_t size = std::max(row, std::min(bytes, kSlotBytes));
+        if (slots_ && n <= nslots_ && size <= slot_bytes_) return hipSuccess;
+        const int want = std::max(n, nslots_);
+        const size_t each = std::max(size, slot_bytes_);
+        if (pinned_) (void)hipHostFree(slots_);
+        else delete[] slots_;
+        nslots_ = 0;
+        slot_bytes_ = 0;
+        slots_ = nullptr;
+        void *p = nullptr;
+        pinned_ = hipHostMalloc(&p, want * each) == hipSuccess;
+        if (!pinned_) (void)hipGetLastError();  // pageable slots work too
+        slots_ = pinned_ ? (char *)p : new (std::nothrow) char[want * each];
+        if (!slots_) return hipErrorOutOfMemory;
+        for (int k = 0; k < want; ++k)
+            if (!done_[k]) {
+                const hipError_t e = hipEventCreateWithFlags(&done_[k], hipEventDisableTiming);
+                if (e != hipSuccess) return e;
+            }
+        nslots_ = want;
+        slot_bytes_ = each;
+        return hipSuccess;
+    }
+
+    // no exception leaves a C entry
+    hipError_t guarded(int device, hipStream_t stream, const Rows &R, const std::vector<Segment> &segs, bool up) {
+        try {
+            return run(device, stream, R, segs, up);
+        } catch (const std::bad_alloc &) {
+            return hipErrorOutOfMemory;
+        }
+    }
+
+    struct Chunk {
+        int seg;
+        long r0, r1;
+    };
+
+    hipError_t run(int device, hipStream_t stream, const Rows &R, const std::vector<Segment> &segs, bool up) {
+        std::lock_guard<std::mutex> hold(lock_);
+        const size_t row = sizeof(double) * (R.length() + 64);  // with the gap behind a field's last row
+        size_t bytes = 0;
+        for (const Segment &s : segs) bytes += sizeof(double) * s.nf * R.fs;
+        if (!bytes) return hipSuccess;
+        hipError_t e = grow(bytes, row);
+        if (e != hipSuccess) return e;
+        std::vector<Chunk> chunks;
+        for (int s = 0; s < (int)segs.size(); ++s) {
+            const long rows = segs[s].nf * R.per_field();
+            const long step = std::max(1L, (long)((slot_bytes_ - 64 * 8) / (sizeof(double) * R.length())));
+            for (long r = 0; r < rows; r += step) {
+                long r1 = std::min(rows, r + step);
+                // the gaps between fields count too
+                while (r1 > r + 1 && sizeof(double) * (R.start(r1) - R.start(r)) > slot_bytes_) --r1;
+                chunks.push_back({s, r, r1});
+                r = r1 - step;
+            }
+        }
+        const int workers = bytes >= kParallelBytes ? kWorkers : 1;
+        hipError_t err[kWorkers] = {};
+        auto work = [&](int w) { err[w] = share(device, stream, R, segs, chunks, w, workers, up); };
+        std::thread helper[kWorkers];
+        for (int w = 1; w < workers; ++w) {
+            try {
+                helper[w] = std::thread(work, w);
+            } catch (...) {  // no thread to be had: this share is done below
+            }
+        }
+        work(0);
+        for (int w = 1; w < workers; ++w) {
+            if (helper[w].joinable()) helper[w].join();
+            else work(w);
+        }
+        e = up ? hipStreamSynchronize(stream) : hipSuccess;
+        for (int w = 0; w < workers; ++w)
+            if (e == hipSuccess) e = err[w];
+        return e;
+    }
+
+    // chunks w, w + workers, ... through slots w * kDepth ..
+    hipError_t share(int device, hipStream_t stream, const Rows &R, const std::vector<Segment> &segs,
+                     const std::vector<Chunk> &chunks, int w, int workers, bool up) {
+        hipError_t e = w ? hipSetDevice(device) : hipSuccess;
+        long issued = 0, taken = 0;  // of this share
+        auto chunk = [&](long n) -> const Chunk * {
+            const size_t at = (size_t)w + (size_t)n * workers;
+            return at < chunks.size() ? &chunks[at] : nullptr;
+        };
+        auto slot = [&](long n) { return (double *)(slots_ + (w * kDepth + n % kDepth) * slot_bytes_); };
+        auto event = [&](long n) { return done_[w * kDepth + n % kDepth]; };
+        while (e == hipSuccess && (chunk(issued) || taken < issued)) {
+            if (const Chunk *c = issued - taken < kDepth ? chunk(issued) : nullptr) {
+                double *dev = segs[c->seg].dev + R.start(c->r0);
+                const size_t n = sizeof(double) * (R.start(c->r1) - R.start(c->r0));
+                if (up) R.in(c->r0, c->r1, segs[c->seg].src, slot(issued));
+                e = up ? hipMemcpyAsync(dev, slot(issued), n, hipMemcpyHostToDevice, stream)
+                       : hipMemcpyAsync(slot(issued), dev, n, hipMemcpyDeviceToHost, stream);
+                if (e == hipSuccess) e = hipEventRecord(event(issued), stream);
+                ++issued;
+                continue;
+            }
+            e = hipEventSynchronize(event(taken));
+            const Chunk *c = chunk(taken);
+            if (e == hipSuccess && !up) R.out(c->r0, c->r1, slot(taken), segs[c->seg].dst);
+            ++taken;
+        }
+        if (e != hipSuccess) (void)hipStreamSynchronize(stream);  // nothing in flight on the slots
+        return e;
+    }
+};
+
+}  // namespace vah_host
