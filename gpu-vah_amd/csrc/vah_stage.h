@@ -220,6 +220,7 @@ __device__ __forceinline__ void face_speeds(double t, double guess2, const R *qR
 // store instead of faulting.  A set must stay below 4 GB (checked on the host).
 // ---------------------------------------------------------------------------
 typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kBufWord3 = 0x00020000;  // raw dword access, gfx9 family
 
@@ -235,6 +236,19 @@ __device__ __forceinline__ Buf make_buf(const double *base, int nfields, long fs
 
 __device__ __forceinline__ double ld(const Buf &b, uint32_t cell, uint32_t field) {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(b.r, (int)cell, (int)field, 0));
+}
+
+// The cell at this offset and the next one in x (16 bytes, 8-byte aligned).  The
+// vector L1 is the busiest unit of the stage kernels (its data return 68 % of the
+// cycles at 611x587, 92 % at 201x201x101) and delivers one such load at 95 bytes per
+// clock, two of 8 bytes at 64, whatever the alignment.  The x stencils and the x
+// differences with their cell loaded this way: 611x587 142 -> 134 us per step,
+// 201x201x101 2.38 -> 2.31 ms, split 97x89x33 173 -> 167 us.
+__device__ __forceinline__ void ld2(const Buf &b, uint32_t cell, uint32_t field, double &v0, double &v1) {
+    const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(b.r, (int)cell, (int)field, 0);
+    const u32x2_t lo = {v.x, v.y}, hi = {v.z, v.w};
+    v0 = __builtin_bit_cast(double, lo);
+    v1 = __builtin_bit_cast(double, hi);
 }
 
 __device__ __forceinline__ void st(const Buf &b, uint32_t cell, uint32_t field, double v) {
@@ -274,8 +288,8 @@ struct AxisFields {  // pi^{DIR mu} for mu = x, y, eta
     static constexpr int n = DIR == 1 ? PIXN : DIR == 2 ? PIYN : PINN;
 };
 
-// Flux through one face.  load(n, j) gives field n at stencil position j
-// (0..3: c-2st .. c+st for the face between cells c-st and c); the left/right
+// Flux through one face.  load(n, v) gives field n at the four stencil positions
+// (c-2st .. c+st for the face between cells c-st and c); the left/right
 // states are the reference's half-cell extrapolations
 // (HalfSiteExtrapolation.cpp:12-26); emit(n, H_n) receives the 15 components in
 // order.  start(guess2, v) loads the solves' start |u_T|^2 and, with AX >= 0,
@@ -291,10 +305,7 @@ __device__ __forceinline__ void face_flux(double t, double h, Start start, Load 
     // all loads of the nine fields first, so that they are in flight together
     double raw[NN][4];
 #pragma unroll
-    for (int n = 0; n < NN; ++n) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) raw[n][j] = load(n, j);
-    }
+    for (int n = 0; n < NN; ++n) load(n, raw[n]);
     // the start (loads of its own) after the stencil loads, so that one wait
     // covers both
     double guess2, v = 0.0;
@@ -323,10 +334,7 @@ __device__ __forceinline__ void face_flux(double t, double h, Start start, Load 
     for (int n = 0; n < NN; ++n) emit(n, cR * qR[n] + cL * qL[n]);
     double rest[NQ - NN][4];
 #pragma unroll
-    for (int n = NN; n < NQ; ++n) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) rest[n - NN][j] = load(n, j);
-    }
+    for (int n = NN; n < NQ; ++n) load(n, rest[n - NN]);
 #pragma unroll
     for (int n = NN; n < NQ; ++n) {
         R q0 = (R)rest[n - NN][0], q1 = (R)rest[n - NN][1], q2 = (R)rest[n - NN][2], q3 = (R)rest[n - NN][3];
@@ -403,29 +411,34 @@ __device__ __forceinline__ void load_src_in(const StageParams &P, const Views &V
     in.t = P.t_src;
     in.dt_inv = P.dt_inv;
     in.etabar_inv = P.etabar_inv;
-    in.e = ld(V.e_in, s, 0);
-    in.p = ld(V.p_in, s, 0);
-    in.ut = ld(u, s, 0);
-    in.ux = ld(u, s, f8);
-    in.uy = ld(u, s, 2 * f8);
-    in.un = ld(u, s, 3 * f8);
+    // The cell together with its left neighbour.  The right neighbours are loaded
+    // below, in the order in which the differences enter the source terms: the
+    // compiler ranks the operands of its sums by their loads, and with them the
+    // products it contracts, which the split precision's float terms would show.
+    double el, pl, utl, uxl, uyl, unl;
+    ld2(V.e_in, s - 8, 0, el, in.e);
+    ld2(V.p_in, s - 8, 0, pl, in.p);
+    ld2(u, s - 8, 0, utl, in.ut);
+    ld2(u, s - 8, f8, uxl, in.ux);
+    ld2(u, s - 8, 2 * f8, uyl, in.uy);
+    ld2(u, s - 8, 3 * f8, unl, in.un);
     in.utp = ld(V.uprev, s, 0);
     in.uxp = ld(V.uprev, s, f8);
     in.uyp = ld(V.uprev, s, 2 * f8);
     in.unp = ld(V.uprev, s, 3 * f8);
     auto cd = [&](const Buf &b, uint32_t fo, uint32_t stp, double h) { return (ld(b, s + stp, fo) - ld(b, s - stp, fo)) * h; };
-    in.dxut = cd(u, 0, 8, P.hx);
-    in.dxux = cd(u, f8, 8, P.hx);
-    in.dxuy = cd(u, 2 * f8, 8, P.hx);
-    in.dxun = cd(u, 3 * f8, 8, P.hx);
+    in.dxut = (ld(u, s + 8, 0) - utl) * P.hx;
+    in.dxux = (ld(u, s + 8, f8) - uxl) * P.hx;
+    in.dxuy = (ld(u, s + 8, 2 * f8) - uyl) * P.hx;
+    in.dxun = (ld(u, s + 8, 3 * f8) - unl) * P.hx;
     in.dyut = cd(u, 0, sy8, P.hy);
     in.dyux = cd(u, f8, sy8, P.hy);
     in.dyuy = cd(u, 2 * f8, sy8, P.hy);
     in.dyun = cd(u, 3 * f8, sy8, P.hy);
     const uint32_t plo = PL * f8;
-    in.dxp = cd(V.p_in, 0, 8, P.hx);
+    in.dxp = (ld(V.p_in, s + 8, 0) - pl) * P.hx;
     in.dyp = cd(V.p_in, 0, sy8, P.hy);
-    in.dxe = cd(V.e_in, 0, 8, P.hx);
+    in.dxe = (ld(V.e_in, s + 8, 0) - el) * P.hx;
     in.dye = cd(V.e_in, 0, sy8, P.hy);
     in.dxpl = cd(V.qin, plo, 8, P.hx);
     in.dypl = cd(V.qin, plo, sy8, P.hy);
@@ -699,7 +712,7 @@ __device__ __forceinline__ void face_role(const StageParams &P, const Views &V, 
             for (int n = 0; n < NQ; ++n) above[n] = ld(V.qin, s + sz8, n * f8);
             face_flux<3, R, true, -1>(
                 t, 0.0, [&](double &guess2, double &) { guess2 = uT2_of(V.ucur, f8, s - sz8); },
-                [&](int n, int j) { return j == 0 ? far[n] : j == 1 ? below[n] : j == 2 ? here[n] : above[n]; },
+                [&](int n, double (&v)[4]) { v[0] = far[n], v[1] = below[n], v[2] = here[n], v[3] = above[n]; },
                 [&](int n, R h) { carry[n] = h; }, [](const R (&)[4]) {});
         }
     }
@@ -708,14 +721,21 @@ __device__ __forceinline__ void face_role(const StageParams &P, const Views &V, 
         if (x_ok) {
             const uint32_t c = cell_offset(P, plane, T.i0 + xi, T.j0 + xj);
             face_flux<1, R, true, 1>(
-                t, P.hx, start(c - 8, c, 1), [&](int n, int j) { return ld(V.qin, c + (uint32_t)j * 8u - 16u, n * f8); },
+                t, P.hx, start(c - 8, c, 1),
+                [&](int n, double (&v)[4]) {
+                    ld2(V.qin, c - 16u, n * f8, v[0], v[1]);
+                    ld2(V.qin, c, n * f8, v[2], v[3]);
+                },
                 [&](int n, R h) { lds.Hx[n][lane] = h; }, axis_to(0));
         }
         const uint32_t s = cell_offset(P, plane, T.i0 + ci, T.j0 + cj);
         if (y_ok) {
             face_flux<2, R, true, 1>(
                 t, P.hy, start(s - sy8, s, 2),
-                [&](int n, int j) { return ld(V.qin, s + (uint32_t)j * sy8 - 2u * sy8, n * f8); },
+                [&](int n, double (&v)[4]) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) v[j] = ld(V.qin, s + (uint32_t)j * sy8 - 2u * sy8, n * f8);
+                },
                 [&](int n, R h) { lds.Hy[n][lane] = h; }, axis_to(1));
         }
         if constexpr (D3) {
@@ -725,7 +745,7 @@ __device__ __forceinline__ void face_role(const StageParams &P, const Views &V, 
                 for (int n = 0; n < NQ; ++n) fresh[n] = ld(V.qin, s + 2u * sz8, n * f8);
                 face_flux<3, R, true, 0>(
                     t, P.hz, start(s, s, 3),
-                    [&](int n, int j) { return j == 0 ? below[n] : j == 1 ? here[n] : j == 2 ? above[n] : fresh[n]; },
+                    [&](int n, double (&v)[4]) { v[0] = below[n], v[1] = here[n], v[2] = above[n], v[3] = fresh[n]; },
                     [&](int n, R h) {
                         lds.Dz[n][lane] = carry[n] - h;
                         carry[n] = h;
@@ -815,7 +835,11 @@ __global__ __launch_bounds__(kCellThreads, kWavesPerSimd) void stage_per_cell_ke
                 auto face = [&](uint32_t c, auto emit) {
                     face_flux<DIR, double, false, -1>(
                         t, 0.0, [&](double &guess2, double &) { guess2 = uTs; },
-                        [&](int n, int j) { return ld(V.qin, c + (uint32_t)j * stp - 2u * stp, n * f8); }, emit,
+                        [&](int n, double (&v)[4]) {
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) v[j] = ld(V.qin, c + (uint32_t)j * stp - 2u * stp, n * f8);
+                        },
+                        emit,
                         [](const double (&)[4]) {});
                 };
                 face(s + stp, [&](int n, double H) { Hs[n][tid] = H; });
