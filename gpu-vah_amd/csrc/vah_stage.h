@@ -195,7 +195,8 @@ __device__ __forceinline__ void face_newton(double t, double guess, const FaceSt
 // paths must end on it, which is everywhere but in failing or barely physical
 // cells; a lane where one of them need not runs the iteration.
 template <int DIR, bool ROOT_JUMP, typename R>
-__device__ __forceinline__ void face_speeds(double t, double guess2, const R *qR, const R *qL, double &vR, double &vL) {
+__device__ __forceinline__ void face_speeds(double t, double guess2, const R *qR, const R *qL, double &vR, double &vL,
+                                            bool live) {
     if (ROOT_JUMP) {
         const FaceStart s = face_start(guess2);
         auto side = [&](const R *q, double *v) {
@@ -204,7 +205,7 @@ __device__ __forceinline__ void face_speeds(double t, double guess2, const R *qR
                                    v);
         };
         const bool okR = side(qR, &vR), okL = side(qL, &vL);
-        if (okR & okL) return;
+        if ((okR & okL) | !live) return;
     }
     auto state = [&](const R *q) {
         return face_state(t, q[TTT], q[TTX], q[TTY], q[TTN], q[PL], q[PITT], q[PITX], q[PITY], q[PITN]);
@@ -296,11 +297,13 @@ struct AxisFields {  // pi^{DIR mu} for mu = x, y, eta
 // the velocity u^DIR / u^tau of the cell whose axis source (SourceTerms.cpp:46-176)
 // is formed on the way: the cell at stencil position AX + 1, whose centred pi
 // differences (times h) are those of positions AX + 2 and AX.  axis(S) receives
-// its four components.  The nine components the recovery needs stay in
+// its four components; a lane that is not live gets some flux without ever
+// iterating.  The nine components the recovery needs stay in
 // registers, the other six are loaded and reconstructed after it, which keeps
 // the live state small.
 template <int DIR, typename R, bool ROOT_JUMP, int AX, typename Start, typename Load, typename Emit, typename Axis>
-__device__ __forceinline__ void face_flux(double t, double h, Start start, Load load, Emit emit, Axis axis) {
+__device__ __forceinline__ void face_flux(double t, double h, Start start, Load load, Emit emit, Axis axis,
+                                          bool live = true) {
     constexpr int NN = 9;  // TTT..PITN
     // all loads of the nine fields first, so that they are in flight together
     double raw[NN][4];
@@ -326,7 +329,7 @@ __device__ __forceinline__ void face_flux(double t, double h, Start start, Load 
     }
     // the recovery of both sides runs in double whatever R is
     double vR, vL;
-    face_speeds<DIR, ROOT_JUMP, R>(t, guess2, qR, qL, vR, vL);
+    face_speeds<DIR, ROOT_JUMP, R>(t, guess2, qR, qL, vR, vL, live);
     const double a = fmax(fabs(vL), fabs(vR));
     // (F(qR) + F(qL) - a (qR - qL)) / 2 with F(q) = v q
     const R cR = (R)(0.5 * (vR - a)), cL = (R)(0.5 * (vL + a));
@@ -669,8 +672,11 @@ __device__ __forceinline__ void cell_role(const StageParams &P, const Views &V, 
 // eta face; the lower one is carried from the plane below.  In 3+1D a lane
 // keeps its column's planes k-1, k, k+1 in registers (90 of the 256; the two
 // x / y solves need about 150), so that an eta face loads one new plane
-// instead of four and the y face takes its own cell from there: 201x201x101
-// 2.68 -> 2.40 ms per step, and the L1 sends a third fewer requests to L2.
+// instead of four: 201x201x101 2.68 -> 2.40 ms per step, and the L1 sends a
+// third fewer requests to L2.  All lanes with a y face keep a column, also the
+// row above the tile, and the y face takes its own cell from it: 2.33 -> 2.28 ms.
+// That row's eta faces are formed with the others and used by no one; its
+// corner ghosts hold no state, so its lanes never enter the iteration (live).
 template <bool D3, typename R, int TX, int TY, int NW>
 __device__ __forceinline__ void face_role(const StageParams &P, const Views &V, const Tile &T, StageLds<D3, R, NW> &lds,
                                           int lane) {
@@ -699,7 +705,7 @@ __device__ __forceinline__ void face_role(const StageParams &P, const Views &V, 
     R carry[NQ];                                              // flux through the lower eta face
     double below[D3 ? NQ : 1], here[D3 ? NQ : 1], above[D3 ? NQ : 1];  // planes k-1, k, k+1 of this column
     if constexpr (D3) {
-        if (z_ok) {
+        if (y_ok) {
             const uint32_t s = cell_offset(P, (uint32_t)plane_of(T.k0, D3) * (uint32_t)P.sz, T.i0 + ci, T.j0 + cj);
             double far[NQ];
 #pragma unroll
@@ -713,7 +719,7 @@ __device__ __forceinline__ void face_role(const StageParams &P, const Views &V, 
             face_flux<3, R, true, -1>(
                 t, 0.0, [&](double &guess2, double &) { guess2 = uT2_of(V.ucur, f8, s - sz8); },
                 [&](int n, double (&v)[4]) { v[0] = far[n], v[1] = below[n], v[2] = here[n], v[3] = above[n]; },
-                [&](int n, R h) { carry[n] = h; }, [](const R (&)[4]) {});
+                [&](int n, R h) { carry[n] = h; }, [](const R (&)[4]) {}, z_ok);
         }
     }
     for (int kk = T.k0; kk < T.k1; ++kk) {
@@ -734,12 +740,15 @@ __device__ __forceinline__ void face_role(const StageParams &P, const Views &V, 
                 t, P.hy, start(s - sy8, s, 2),
                 [&](int n, double (&v)[4]) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) v[j] = ld(V.qin, s + (uint32_t)j * sy8 - 2u * sy8, n * f8);
+                    for (int j = 0; j < 4; ++j) {
+                        if (D3 && j == 2) v[j] = here[n];
+                        else v[j] = ld(V.qin, s + (uint32_t)j * sy8 - 2u * sy8, n * f8);
+                    }
                 },
                 [&](int n, R h) { lds.Hy[n][lane] = h; }, axis_to(1));
         }
         if constexpr (D3) {
-            if (z_ok) {
+            if (y_ok) {
                 double fresh[NQ];
 #pragma unroll
                 for (int n = 0; n < NQ; ++n) fresh[n] = ld(V.qin, s + 2u * sz8, n * f8);
@@ -750,7 +759,7 @@ __device__ __forceinline__ void face_role(const StageParams &P, const Views &V, 
                         lds.Dz[n][lane] = carry[n] - h;
                         carry[n] = h;
                     },
-                    axis_to(2));
+                    axis_to(2), z_ok);
 #pragma unroll
                 for (int n = 0; n < NQ; ++n) {
                     below[n] = here[n];
