@@ -44,6 +44,13 @@ constexpr int kTileX = 8;
 constexpr int kTileY = 7;
 constexpr int kTileWaves = 1;  // waves per role
 
+// Tile of the single-lattice kernels on large 3+1D lattices: 16 x 7 cells, two
+// waves per role.  A field's row with its halo is 20 doubles, 2.2 lines of 128 bytes
+// on average, where two tiles of 8 x 7 need 1.7 each (choose_wide_tiles says where
+// that pays).
+constexpr int kWideTileX = 16;
+constexpr int kWideTileWaves = 2;
+
 // The per-cell-flux kernels: 256 lanes, one per cell of a 16 x 16 tile.
 constexpr int kCellTileX = 16;
 constexpr int kCellTileY = 16;
@@ -802,14 +809,14 @@ __device__ __forceinline__ const StageParams &kernarg_params() {
 }
 
 // One event: workgroup -> tile (XCD-aware) -> stage_tile.
-template <bool D3, bool STAGE2, typename R>
-__global__ __launch_bounds__(128 * kTileWaves, kWavesPerSimd) void stage_kernel(StageParams P_arg) {
+template <bool D3, bool STAGE2, typename R, int TX, int NW>
+__global__ __launch_bounds__(128 * NW, kWavesPerSimd) void stage_kernel(StageParams P_arg) {
     const StageParams &P = kernarg_params();
     (void)P_arg;
-    __shared__ StageLds<D3, R, kTileWaves> lds;
+    __shared__ StageLds<D3, R, NW> lds;
     const int tile = tile_of_block(P, (int)blockIdx.x);
     if (tile < 0) return;  // padding workgroups: no barrier reached
-    stage_tile<D3, STAGE2, R, kTileX, kTileY, kTileWaves>(P, tile, lds);
+    stage_tile<D3, STAGE2, R, TX, kTileY, NW>(P, tile, lds);
 }
 
 // The reference's work split (VAH_FLUX_PER_CELL): a lane per cell solves both of
@@ -908,6 +915,7 @@ struct StageLaunch {
     int grid;
     hipStream_t stream;
     int precision, flux_mode;
+    bool wide;  // 16 x 7 tiles
 };
 void launch_stage_3d(const StageLaunch &L, int stage, const StageParams &P);
 
