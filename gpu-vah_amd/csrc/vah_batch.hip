@@ -54,9 +54,10 @@ struct Variant {
 };
 
 // Tile shapes and eta chunks the autotuner chooses from.  64 boost-invariant
-// events of side 101-261 take 0.98 / 1.01 / 1.00 / 1.03 / 1.03 ms per step with
-// them in this order, a few events (whose tiles do not fill the chip) least
-// with the smallest tile, which is the default.
+// events of side 101-261 take 0.88 / 0.92 / 0.92 / 0.91 / 0.91 ms per step with
+// them in this order, three 3+1D events of side 121-181 2.41 / 2.47 / 2.37 / 2.38 /
+// 2.33; a few events (whose tiles do not fill the chip) least with the smallest
+// tile, which is the default.
 const Variant kVariants[] = {
     {{16, 15, kWavesPerSimd, 3}, 4, batch_stage_t16x15},
     {{8, 7, kWavesPerSimd, 3}, 1, batch_stage_t8x7},
