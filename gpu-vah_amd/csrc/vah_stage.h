@@ -909,7 +909,7 @@ inline dim3 ghost_grid(int nx, int ny, int nz) {
 }
 
 // The launches of the 3+1D stage kernels (vah_stage3d.hip): a translation
-// unit of their own, compiled with the scheduler settings that suit them.
+// unit of their own.
 // precision and flux_mode take the values of include/vah.h.
 struct StageLaunch {
     int grid;

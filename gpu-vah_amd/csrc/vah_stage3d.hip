@@ -1,8 +1,5 @@
-// vah_stage3d.hip -- launches of the 3+1D single-lattice stage kernels.  They
-// sit in a translation unit of their own because the machine scheduler with
-// the AMDGPU register-pressure trackers (-amdgpu-use-amdgpu-trackers) speeds
-// them up (201x201x101 FP64 step 2.61 -> 2.56 ms) but slows the 2+1D kernels
-// (81x81 step 0.0756 -> 0.0794 ms); the build gives this unit that setting only.
+// vah_stage3d.hip -- launches of the 3+1D single-lattice stage kernels, a translation
+// unit of their own so that they compile beside the 2+1D ones.
 #include <hip/hip_runtime.h>
 
 #include "../../include/vah.h"
