@@ -467,6 +467,7 @@ void vah_batch_destroy(vah_batch *b) {
         if (st.host) (void)hipHostFree(st.host);
         if (st.done) (void)hipEventDestroy(st.done);
     }
+    b->transfer.release();
     if (b->own_stream && b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
 }

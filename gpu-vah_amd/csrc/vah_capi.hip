@@ -749,8 +749,6 @@ int vah_create(const vah_lattice *lat, const vah_hydro *hydro, const vah_options
         c->grid = g.grid;
         c->wide = g.wide;
     }
-    if (c->transfer.reserve(sizeof(double) * 25 * c->fs, sizeof(double) * (c->ncx + 64)) != hipSuccess)
-        return cleanup(fail(VAH_ERR_NOMEM, "vah_create: transfer slots"));
     c->red_blocks = 1024;
     if (hipMalloc(&c->red_buf, sizeof(double) * 4 * c->red_blocks) != hipSuccess)
         return cleanup(fail(VAH_ERR_NOMEM, "vah_create: reduction buffer"));
@@ -770,6 +768,7 @@ void vah_destroy(vah_ctx *c) {
     (void)hipFree(c->powf_fix);
     (void)hipFree(c->eos_dev);
     (void)hipFree(c->red_buf);
+    c->transfer.release();
     if (c->own_stream && c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }

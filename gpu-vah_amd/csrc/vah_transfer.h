@@ -4,12 +4,12 @@
 // What bounds a transfer is the host side: e, p and u of 201x201x101 cells (196 MB)
 // were copied whole into a pageable buffer, its pages touched for the first time,
 // then picked out of it cell by cell with two divisions per element, and took 130 of
-// the 226 ms of an output interval of 40 steps (97 ms now).  A checkpoint of 201x201
-// cells (25 fields up, 30 down) went from 6.9 to 1.5 ms.
-// Here chunks of at most kSlotBytes go through pinned slots, whole rows are copied
-// between a slot and the caller's array while the next chunk is on the link, and
-// from kParallelBytes on kWorkers host threads share the chunks (one thread copies
-// rows at about 10 GB/s, a fifth of the link).
+// the 226 ms of an output interval of 40 steps (97 ms with the same kernels).  A
+// checkpoint of 201x201 cells (25 fields up, 30 down) went from 6.9 to 1.5 ms.
+// Here chunks of at most kSlotBytes go through slots that the owner keeps, pinned from
+// kPinnedBytes on; whole rows are copied between a slot and the caller's array while
+// the next chunk is on the link; and from kParallelBytes on kWorkers host threads share
+// the chunks (one thread copies rows at about 10 GB/s, a fifth of the link).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -73,14 +73,28 @@ struct Segment {
     const double *src;
 };
 
-// Pinned slots of one context or batch.  Transfers on one object from several
+// The slots of one context or batch.  Transfers on one object from several
 // threads take turns.
 class Transfer {
   public:
     ~Transfer() { release(); }
 
-    // Slots for transfers of up to `bytes` in rows of `row` bytes: called when the
-    // owner is created, and again by transfers that need more.
+    // Called before the owner destroys the stream the events were recorded on.
+    void release() {
+        for (hipEvent_t &e : done_)
+            if (e) {
+                (void)hipEventDestroy(e);
+                e = nullptr;
+            }
+        if (pinned_) (void)hipHostFree(slots_);
+        else delete[] slots_;
+        slots_ = nullptr;
+        pinned_ = false;
+        nslots_ = 0;
+        slot_bytes_ = 0;
+    }
+
+    // Slots for transfers of up to `bytes` in rows of `row` bytes ahead of the first.
     hipError_t reserve(size_t bytes, size_t row) {
         std::lock_guard<std::mutex> hold(lock_);
         return grow(bytes, row);
@@ -93,31 +107,29 @@ class Transfer {
     }
 
   private:
-    static constexpr size_t kSlotBytes = 2 << 20;
+    static constexpr size_t kSlotBytes = 1 << 20;
+    // Below this a context that lives for one short event would pay more for pinned
+    // slots and their events than it saves: create, set, one step, read and close of
+    // 41x37 cells 0.88 ms with them, 0.47 ms with pageable slots and one wait per chunk
+    // (0.73 ms before).  From here on they pay: a checkpoint of 201x201 cells 1.45 ms,
+    // 1.95 ms pageable; the whole life of such a context 3.8 ms (9.8 ms before).
+    static constexpr size_t kPinnedBytes = 4 << 20;
     static constexpr size_t kParallelBytes = 16 << 20;  // below, starting threads costs what they save
     static constexpr int kWorkers = 4, kDepth = 2;      // slots per worker: one on the link, one being copied
 
     std::mutex lock_;
     char *slots_ = nullptr;
-    bool pinned_ = false;
+    bool pinned_ = false, refused_ = false;
     int nslots_ = 0;
     size_t slot_bytes_ = 0;
     hipEvent_t done_[kWorkers * kDepth] = {};
 
-    void release() {
-        for (hipEvent_t &e : done_)
-            if (e) (void)hipEventDestroy(e);
-        if (pinned_) (void)hipHostFree(slots_);
-        else delete[] slots_;
-        slots_ = nullptr;
-        nslots_ = 0;
-        slot_bytes_ = 0;
-    }
-
     hipError_t grow(size_t bytes, size_t row) {
         const int n = kDepth * (bytes >= kParallelBytes ? kWorkers : 1);
         const size_t size = std::max(row, std::min(bytes, kSlotBytes));
-        if (slots_ && n <= nslots_ && size <= slot_bytes_) return hipSuccess;
+        const bool pin = pinned_ || bytes >= kPinnedBytes;
+        if (slots_ && n <= nslots_ && size <= slot_bytes_ && (!pin || pinned_ || refused_))
+            return hipSuccess;
         const int want = std::max(n, nslots_);
         const size_t each = std::max(size, slot_bytes_);
         if (pinned_) (void)hipHostFree(slots_);
@@ -126,11 +138,14 @@ class Transfer {
         slot_bytes_ = 0;
         slots_ = nullptr;
         void *p = nullptr;
-        pinned_ = hipHostMalloc(&p, want * each) == hipSuccess;
-        if (!pinned_) (void)hipGetLastError();  // pageable slots work too
+        pinned_ = pin && !refused_ && hipHostMalloc(&p, want * each) == hipSuccess;
+        if (pin && !pinned_) {  // pageable slots work too
+            refused_ = true;
+            (void)hipGetLastError();
+        }
         slots_ = pinned_ ? (char *)p : new (std::nothrow) char[want * each];
         if (!slots_) return hipErrorOutOfMemory;
-        for (int k = 0; k < want; ++k)
+        for (int k = 0; pinned_ && k < want; ++k)
             if (!done_[k]) {
                 const hipError_t e = hipEventCreateWithFlags(&done_[k], hipEventDisableTiming);
                 if (e != hipSuccess) return e;
@@ -189,7 +204,7 @@ class Transfer {
             if (helper[w].joinable()) helper[w].join();
             else work(w);
         }
-        e = up ? hipStreamSynchronize(stream) : hipSuccess;
+        e = hipStreamSynchronize(stream);
         for (int w = 0; w < workers; ++w)
             if (e == hipSuccess) e = err[w];
         return e;
@@ -213,11 +228,11 @@ class Transfer {
                 if (up) R.in(c->r0, c->r1, segs[c->seg].src, slot(issued));
                 e = up ? hipMemcpyAsync(dev, slot(issued), n, hipMemcpyHostToDevice, stream)
                        : hipMemcpyAsync(slot(issued), dev, n, hipMemcpyDeviceToHost, stream);
-                if (e == hipSuccess) e = hipEventRecord(event(issued), stream);
+                if (e == hipSuccess) e = pinned_ ? hipEventRecord(event(issued), stream) : hipStreamSynchronize(stream);
                 ++issued;
                 continue;
             }
-            e = hipEventSynchronize(event(taken));
+            if (pinned_) e = hipEventSynchronize(event(taken));
             const Chunk *c = chunk(taken);
             if (e == hipSuccess && !up) R.out(c->r0, c->r1, slot(taken), segs[c->seg].dst);
             ++taken;
