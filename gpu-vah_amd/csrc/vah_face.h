@@ -22,9 +22,11 @@
 //       leave [0, u*]; every later one climbs towards the root.
 // (c) needs no division: u1 = u0 - f/f' >= eps u0  <=>  f <= (1 - eps) u0 f',
 // and u0 f' = U0 (B - U0 xM) / (1 + u0^2).  The tests keep a margin of 1e-9,
-// far above rounding.  A state that fails one of them (an unphysical or NaN
-// state, or a path that may fall back) gets `false`, and the caller runs the
-// reference's iteration; every decision is then the full path's.
+// far above rounding.  B < 1e140 as well, so that its square does not overflow; the
+// floor of sqrt_coarse keeps it above 1.5e-140, where the root's square is far above
+// its own floor.  A state that fails one of the tests (an unphysical or NaN state, or a
+// path that may fall back) gets `false`, and the caller runs the reference's iteration;
+// every decision is then the full path's.
 //
 // The root gives the speed without its square roots and quotients by M_T:
 //     v = U* x M^DIR / M_T = 2 x^2 M^DIR / (B + sqrt(B^2 - 2 xM^2)),
@@ -38,9 +40,10 @@
 
 namespace vah {
 
-// sqrt(x) for x >= 0 to about 2^-45, for the tests only (their margin is 1e-9)
+// sqrt(x) for x >= 0 to about 2^-45, at least 1e-140, for the tests only (their margin
+// is 1e-9)
 __host__ __device__ inline double sqrt_coarse(double x) {
-    const double m = __builtin_fmax(x, 1e-300);
+    const double m = __builtin_fmax(x, 1e-280);
     const double y = rsq_estimate(m), g = m * y;
     return __builtin_fma(__builtin_fma(-g, g, m), 0.5 * y, g);
 }
@@ -82,7 +85,8 @@ __host__ __device__ inline FaceSetup face_setup(double t, double M0, double M1, 
     r.B = __builtin_fma(0.5, r.c0 - PL, bL);
     const double f0 = __builtin_fma(s.U0, __builtin_fma(-0.5 * s.U0, xM, r.B), -xM);
     const double h = s.U0 * s.w * __builtin_fma(-s.U0, xM, r.B);
-    r.ok = (Ft2 < 1.0 - 1e-6) & (r.B > 1.5 * kMargin * xM) & (r.c0 > kMargin * xM) & (f0 <= (1.0 - 1e-9) * h);
+    r.ok = (Ft2 < 1.0 - 1e-6) & (r.B > 1.5 * kMargin * xM) & (r.B < 1e140) & (r.c0 > kMargin * xM) &
+           (f0 <= (1.0 - 1e-9) * h);
     return r;
 }
 
