@@ -5,12 +5,17 @@
 
 namespace vah {
 
-// hardware estimates on the device, the plain quotients on the host
+// The hardware estimates on the device (relative error up to 2^-23); on the host the
+// plain quotients, which a test build can put off by as much through VAH_SEED.
+#ifndef VAH_SEED
+#define VAH_SEED(s) (s)
+#endif
+
 __host__ __device__ inline double rcp_estimate(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
     return __builtin_amdgcn_rcp(x);
 #else
-    return 1.0 / x;
+    return VAH_SEED(1.0 / x);
 #endif
 }
 
@@ -18,7 +23,7 @@ __host__ __device__ inline double rsq_estimate(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
     return __builtin_amdgcn_rsq(x);
 #else
-    return 1.0 / __builtin_sqrt(x);
+    return VAH_SEED(1.0 / __builtin_sqrt(x));
 #endif
 }
 

@@ -40,7 +40,7 @@
 
 namespace vah {
 
-// sqrt(x) for x >= 0 to about 2^-45, at least 1e-140, for the tests only (their margin
+// sqrt(x) for x >= 0 to 2^-43, at least 1e-140, for the tests only (their margin
 // is 1e-9)
 __host__ __device__ inline double sqrt_coarse(double x) {
     const double m = __builtin_fmax(x, 1e-280);
