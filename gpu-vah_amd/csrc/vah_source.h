@@ -306,7 +306,8 @@ __device__ __forceinline__ void regulate(double t, const Eos &E, const EosP &pe,
     // ratios to spipi; a zero spipi makes them 0 * inf = NaN (or +-inf for a
     // nonzero numerator), as the quotients would be
     const double pipi2 = fabs(pipi);
-    double ispipi = rsqrt(pipi2), spipi = pipi2 * ispipi;
+    const Root rpipi = root_of(pipi2);
+    double ispipi = rpipi.inverse, spipi = rpipi.root;
     if (!(pipi2 > 1e-280 && pipi2 < 1e280)) {
         spipi = __builtin_sqrt(pipi2);
         ispipi = 1.0 / spipi;
@@ -318,7 +319,7 @@ __device__ __forceinline__ void regulate(double t, const Eos &E, const EosP &pe,
     if (floor_e) p = 1.e-7;
     const double ptHat = 0.5 * ((e - pl) - rb * (e - 3.0 * p));
     const double s2 = fabs(e * e + pl * pl + 2.0 * ptHat * ptHat);
-    double rho = spipi * rsqrt(s2);
+    double rho = quotient(spipi, root_of(s2));
     if (!(s2 > 1e-280 && s2 < 1e280)) rho = spipi / __builtin_sqrt(s2);
     if (am > rho) rho = am;
     double fac = tanh_over_x(rho);  // tanh(rho) / rho
