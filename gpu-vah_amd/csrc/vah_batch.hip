@@ -54,18 +54,21 @@ struct Variant {
 };
 
 // Tile shapes and eta chunks the autotuner chooses from.  64 boost-invariant
-// events of side 101-261 take 0.88 / 0.92 / 0.92 / 0.91 / 0.91 ms per step with
-// them in this order, three 3+1D events of side 121-181 2.41 / 2.47 / 2.37 / 2.38 /
-// 2.33; a few events (whose tiles do not fill the chip) least with the smallest
-// tile, which is the default.
+// events of side 101-261 take 0.88 / 0.91 / 0.92 ms per step with 16 x 15, 16 x 7 and
+// 8 x 7 tiles, three 3+1D events of side 121-181 2.41 / 2.38 / 2.47 with three planes
+// and, with six, 2.33 in 16 x 7 and 2.37 in 8 x 7; a few events (whose tiles do not
+// fill the chip) least with the smallest tile, which is the default.
+// Callers may have stored an index: 0 and 1 keep their tile and chunk, 2 to 5 are the
+// shapes that took the places of 32 x 7 tiles and of a third workgroup per CU.
 const Variant kVariants[] = {
     {{16, 15, kWavesPerSimd, 3}, 4, batch_stage_t16x15},
-    {{8, 7, kWavesPerSimd, 3}, 1, batch_stage_t8x7},
-    {{8, 7, kWavesPerSimd, 6}, 1, batch_stage_t8x7},
+    {{16, 15, kWavesPerSimd, 6}, 4, batch_stage_t16x15},
     {{16, 7, kWavesPerSimd, 3}, 2, batch_stage_t16x7},
     {{16, 7, kWavesPerSimd, 6}, 2, batch_stage_t16x7},
+    {{8, 7, kWavesPerSimd, 3}, 1, batch_stage_t8x7},
+    {{8, 7, kWavesPerSimd, 6}, 1, batch_stage_t8x7},
 };
-constexpr int kDefaultVariant = 1;
+constexpr int kDefaultVariant = 4;
 constexpr int kNumVariants = (int)(sizeof kVariants / sizeof kVariants[0]);
 
 struct HostEvent {

@@ -139,7 +139,9 @@ int vah_batch_retire(vah_batch *b, int slot);
 int vah_batch_memory(const vah_batch *b, size_t *used, size_t *budget);
 
 /* Kernel variants: tile shape, occupancy target and eta-chunk.  Every
- * variant computes the same per-cell arithmetic. */
+ * variant computes the same per-cell arithmetic.  Choose one by what
+ * vah_batch_variant_info says rather than by a stored index: indices 0 to 5 stay
+ * valid, but 2 to 5 do not name the kernels they first did. */
 int vah_batch_variant_count(void);
 int vah_batch_variant_info(int index, vah_batch_variant *out);
 int vah_batch_set_variant(vah_batch *b, int index);
