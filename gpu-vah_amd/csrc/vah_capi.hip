@@ -181,54 +181,8 @@ bool lattice_ok(const vah_lattice *l) {
     return l && l->nx > 0 && l->ny > 0 && l->nz > 0 && l->dx > 0 && l->dy > 0 && l->dz > 0 && l->dt > 0;
 }
 
-// Launch geometry of one lattice: tiles marching kz eta planes.
-struct Geometry {
-    int tiles_x, tiles_y, zchunks, kz, nblocks, grid;
-    bool wide;  // 16 x 7 tiles instead of 8 x 7
-};
-
-// Eta planes per workgroup when the caller leaves the choice (opt.eta_chunk 0).
-// A chunk of kz planes solves kz + 1 eta faces per cell and starts by loading
-// three planes of each column, so longer chunks do less work; but a lattice of
-// few tiles then leaves CUs idle.  About 1,024 workgroups (four per CU) run at
-// once.  Measured per pass with kz = 1 / 3 / 6: 53x67x13 (70 tiles) 192 / 281 /
-// 424 us, 101x101x30 (195 tiles) 830 / 775 / 775 us, 201x201x101 (754 tiles)
-// 2.62 / 2.41 / 2.40 ms per step (12: 2.49).
-int choose_eta_chunk(int tiles, int nz, bool wide) {
-    auto groups = [&](int kz) { return (long)tiles * ((nz + kz - 1) / kz); };
-    if (wide) return groups(6) >= 2048 ? 6 : 3;
-    if (groups(6) >= 4096) return 6;
-    if (groups(3) >= 1536) return 3;
-    if (groups(2) >= 1536) return 2;
-    return 1;
-}
-
-// 16 x 7 tiles pay where the lattice gives about 2,300 workgroups of three planes:
-// 512 of them run at once, and with fewer than some four rounds the last one, of
-// workgroups twice as long, costs more than the halo saves.  Per step with 8 x 7 /
-// 16 x 7 tiles, FP64: 101x101x30 (1,050 workgroups) 190 / 206 us, 101x101x60 (2,100)
-// 385 / 391, 121x121x50 (2,448) 473 / 457, 151x151x101 1322 / 1200, 201x201x101
-// 2267 / 2024, 301x301x31 1597 / 1398; split 101x101x60 379 / 379, 121x121x50
-// 459 / 440, 201x201x101 2243 / 1986.  Tiles of 16 x 15 (four waves per role):
-// 2238 at 201x201x101; 2+1D at 611x587: 133 / 140.
-bool choose_wide_tiles(const vah_lattice &lat) {
-    const long tiles = (long)((lat.nx + kWideTileX - 1) / kWideTileX) * ((lat.ny + kTileY - 1) / kTileY);
-    return lat.nz > 1 && tiles * ((lat.nz + 2) / 3) >= 2300;
-}
-
 Geometry make_geometry(const vah_lattice &lat, int flux_mode, int eta_chunk) {
-    const bool shared = flux_mode == VAH_FLUX_SHARED;
-    Geometry g;
-    g.wide = shared && choose_wide_tiles(lat);
-    const int tx = !shared ? kCellTileX : g.wide ? kWideTileX : kTileX, ty = shared ? kTileY : kCellTileY;
-    g.tiles_x = (lat.nx + tx - 1) / tx;
-    g.tiles_y = (lat.ny + ty - 1) / ty;
-    const int tiles = g.tiles_x * g.tiles_y;
-    g.kz = lat.nz > 1 ? std::min(eta_chunk > 0 ? eta_chunk : choose_eta_chunk(tiles, lat.nz, g.wide), lat.nz) : 1;
-    g.zchunks = (lat.nz + g.kz - 1) / g.kz;
-    g.nblocks = tiles * g.zchunks;
-    g.grid = g.zchunks * 8 * ((tiles + 7) / 8);  // tile_of_block's grid
-    return g;
+    return launch_geometry(lat.nx, lat.ny, lat.nz, flux_mode == VAH_FLUX_SHARED, eta_chunk);
 }
 
 // Everything of a stage's parameters except its buffers and times.
@@ -359,7 +313,7 @@ void launch_variant(const LaunchCfg &L, const StageParams &P) {
         hipLaunchKernelGGL((stage_per_cell_kernel<false, S2>), dim3(L.grid), dim3(kCellThreads), 0, L.stream, P);
 }
 
-// 2+1D here; 3+1D in vah_stage3d.hip (compiled with other scheduler settings)
+// 2+1D here; 3+1D in vah_stage3d.hip
 void launch_stage(const LaunchCfg &L, int stage, const StageParams &P) {
     if (L.d3) {
         launch_stage_3d(StageLaunch{L.grid, L.stream, L.precision, L.flux_mode, L.wide}, stage, P);

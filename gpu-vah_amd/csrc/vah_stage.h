@@ -33,28 +33,10 @@
 
 #include "vah_device.h"
 #include "vah_face.h"
+#include "vah_geometry.h"
 #include "vah_source.h"
 
 namespace vah {
-
-// Tile of the single-lattice kernels: 8 x 7 cells, one face wave and one cell
-// wave.  Its x faces (9 x 7 = 63) and y faces (8 x 8 = 64) fill a wave, its
-// cells 56 lanes of one.
-constexpr int kTileX = 8;
-constexpr int kTileY = 7;
-constexpr int kTileWaves = 1;  // waves per role
-
-// Tile of the single-lattice kernels on large 3+1D lattices: 16 x 7 cells, two
-// waves per role.  A field's row with its halo is 20 doubles, 2.2 lines of 128 bytes
-// on average, where two tiles of 8 x 7 need 1.7 each (choose_wide_tiles says where
-// that pays).
-constexpr int kWideTileX = 16;
-constexpr int kWideTileWaves = 2;
-
-// The per-cell-flux kernels: 256 lanes, one per cell of a 16 x 16 tile.
-constexpr int kCellTileX = 16;
-constexpr int kCellTileY = 16;
-constexpr int kCellThreads = 256;
 
 // Waves per SIMD the register allocation is sized for: 512 registers shared by
 // two leave 256 to each.  At three (168 each) the source terms spill and every
