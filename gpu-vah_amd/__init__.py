@@ -431,7 +431,7 @@ def batch_event_bytes(nx, ny, nz):
 
 
 def batch_variants():
-    """The compiled kernel variants: (tile_x, tile_y, blocks_per_cu, kz)."""
+    """The compiled kernel variants: (tile_x, tile_y, groups of 256 lanes per CU, kz)."""
     out = []
     for i in range(lib().vah_batch_variant_count()):
         v = BatchVariant()

@@ -6,8 +6,8 @@
 // then picked out of it cell by cell with two divisions per element, and took 130 of
 // the 226 ms of an output interval of 40 steps (97 ms with the same kernels).  A
 // checkpoint of 201x201 cells (25 fields up, 30 down) went from 6.9 to 1.5 ms.
-// Here chunks of at most kSlotBytes go through slots that the owner keeps, pinned from
-// kPinnedBytes on; whole rows are copied between a slot and the caller's array while
+// Here chunks of whole rows, at most kSlotBytes (or one row, where it is longer), go
+// through slots that the owner keeps, pinned from kPinnedBytes on; whole rows are copied between a slot and the caller's array while
 // the next chunk is on the link; and from kParallelBytes on kWorkers host threads share
 // the chunks (one thread copies rows at about 10 GB/s, a fifth of the link).
 #pragma once

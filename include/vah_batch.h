@@ -81,7 +81,9 @@ typedef struct vah_batch_status {
 
 typedef struct vah_batch_variant {
     int tile_x, tile_y;        /* cells per workgroup tile */
-    int blocks_per_cu;         /* waves per SIMD the registers are sized for */
+    int blocks_per_cu;         /* groups of 256 lanes (a wave per SIMD) per CU that the registers are sized for;
+                                * in workgroups of the tile: 16 x 15 (512 lanes) half as many, 16 x 7 (256)
+                                * as many, 8 x 7 (128) twice as many */
     int kz;                    /* eta planes per 3+1D tile */
 } vah_batch_variant;
 
