@@ -5,11 +5,12 @@
 // were copied whole into a pageable buffer, its pages touched for the first time,
 // then picked out of it cell by cell with two divisions per element, and took 130 of
 // the 226 ms of an output interval of 40 steps (97 ms with the same kernels).  A
-// checkpoint of 201x201 cells (25 fields up, 30 down) went from 6.9 to 1.5 ms.
+// checkpoint of 201x201 cells (25 fields up, 30 down) went from 6.9 to 1.34 ms.
 // Here chunks of whole rows, at most kSlotBytes (or one row, where it is longer), go
-// through slots that the owner keeps, pinned from kPinnedBytes on; whole rows are copied between a slot and the caller's array while
-// the next chunk is on the link; and from kParallelBytes on kWorkers host threads share
-// the chunks (one thread copies rows at about 10 GB/s, a fifth of the link).
+// through slots that the owner keeps, pinned from kPinnedBytes on; rows are copied
+// between a slot and the caller's array while the next chunk is on the link; and from
+// kParallelBytes on kWorkers host threads share the chunks (one thread copies rows at
+// about 10 GB/s, a fifth of the link).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -79,13 +80,7 @@ class Transfer {
   public:
     ~Transfer() { release(); }
 
-    // Called before the owner destroys the stream the events were recorded on.
     void release() {
-        for (hipEvent_t &e : done_)
-            if (e) {
-                (void)hipEventDestroy(e);
-                e = nullptr;
-            }
         if (pinned_) (void)hipHostFree(slots_);
         else delete[] slots_;
         slots_ = nullptr;
@@ -109,10 +104,10 @@ class Transfer {
   private:
     static constexpr size_t kSlotBytes = 1 << 20;
     // Below this a context that lives for one short event would pay more for pinned
-    // slots and their events than it saves: create, set, one step, read and close of
-    // 41x37 cells 0.88 ms with them, 0.47 ms with pageable slots and one wait per chunk
-    // (0.73 ms before).  From here on they pay: a checkpoint of 201x201 cells 1.45 ms,
-    // 1.95 ms pageable; the whole life of such a context 3.8 ms (9.8 ms before).
+    // slots than it saves: create, set, one step, read and close of 41x37 cells 0.88 ms
+    // with them, 0.47 ms with pageable slots (0.73 ms before).  From here on they pay: a
+    // checkpoint of 201x201 cells 1.45 ms, 1.95 ms pageable, when both were measured; the
+    // whole life of such a context takes 1.35 ms (9.8 ms before).
     static constexpr size_t kPinnedBytes = 4 << 20;
     static constexpr size_t kParallelBytes = 16 << 20;  // below, starting threads costs what they save
     static constexpr int kWorkers = 4, kDepth = 2;      // slots per worker: one on the link, one being copied
@@ -122,7 +117,6 @@ class Transfer {
     bool pinned_ = false, refused_ = false;
     int nslots_ = 0;
     size_t slot_bytes_ = 0;
-    hipEvent_t done_[kWorkers * kDepth] = {};
 
     hipError_t grow(size_t bytes, size_t row) {
         const int n = kDepth * (bytes >= kParallelBytes ? kWorkers : 1);
@@ -145,11 +139,6 @@ class Transfer {
         }
         slots_ = pinned_ ? (char *)p : new (std::nothrow) char[want * each];
         if (!slots_) return hipErrorOutOfMemory;
-        for (int k = 0; pinned_ && k < want; ++k)
-            if (!done_[k]) {
-                const hipError_t e = hipEventCreateWithFlags(&done_[k], hipEventDisableTiming);
-                if (e != hipSuccess) return e;
-            }
         nslots_ = want;
         slot_bytes_ = each;
         return hipSuccess;
@@ -210,32 +199,35 @@ class Transfer {
         return e;
     }
 
-    // chunks w, w + workers, ... through slots w * kDepth ..
+    // Chunks w, w + workers, ... through two slots: one copy of this share is on the link
+    // while the host copies the chunk before it (down) or after it (up).  Waits are for
+    // the stream: with an event per chunk, waited for, the runtime took 0.7 to 2.8 ms
+    // longer over the next stream, allocation and pageable copy of the process (creating
+    // the next context of 201x201 cells 0.26 -> 2.6 ms), however the events were made or
+    // kept; recorded but not waited for they cost nothing.
     hipError_t share(int device, hipStream_t stream, const Rows &R, const std::vector<Segment> &segs,
                      const std::vector<Chunk> &chunks, int w, int workers, bool up) {
         hipError_t e = w ? hipSetDevice(device) : hipSuccess;
-        long issued = 0, taken = 0;  // of this share
-        auto chunk = [&](long n) -> const Chunk * {
-            const size_t at = (size_t)w + (size_t)n * workers;
-            return at < chunks.size() ? &chunks[at] : nullptr;
+        auto slot = [&](size_t n) { return (double *)(slots_ + (w * kDepth + n / workers % kDepth) * slot_bytes_); };
+        auto copy = [&](size_t n) {
+            const Chunk &c = chunks[n];
+            double *dev = segs[c.seg].dev + R.start(c.r0);
+            const size_t bytes = sizeof(double) * (R.start(c.r1) - R.start(c.r0));
+            return up ? hipMemcpyAsync(dev, slot(n), bytes, hipMemcpyHostToDevice, stream)
+                      : hipMemcpyAsync(slot(n), dev, bytes, hipMemcpyDeviceToHost, stream);
         };
-        auto slot = [&](long n) { return (double *)(slots_ + (w * kDepth + n % kDepth) * slot_bytes_); };
-        auto event = [&](long n) { return done_[w * kDepth + n % kDepth]; };
-        while (e == hipSuccess && (chunk(issued) || taken < issued)) {
-            if (const Chunk *c = issued - taken < kDepth ? chunk(issued) : nullptr) {
-                double *dev = segs[c->seg].dev + R.start(c->r0);
-                const size_t n = sizeof(double) * (R.start(c->r1) - R.start(c->r0));
-                if (up) R.in(c->r0, c->r1, segs[c->seg].src, slot(issued));
-                e = up ? hipMemcpyAsync(dev, slot(issued), n, hipMemcpyHostToDevice, stream)
-                       : hipMemcpyAsync(slot(issued), dev, n, hipMemcpyDeviceToHost, stream);
-                if (e == hipSuccess) e = pinned_ ? hipEventRecord(event(issued), stream) : hipStreamSynchronize(stream);
-                ++issued;
+        if (!up && e == hipSuccess && (size_t)w < chunks.size()) e = copy(w);
+        for (size_t n = w; e == hipSuccess && n < chunks.size(); n += workers) {
+            const Chunk &c = chunks[n];
+            if (up) {
+                R.in(c.r0, c.r1, segs[c.seg].src, slot(n));
+                if (n >= (size_t)workers) e = hipStreamSynchronize(stream);  // the other slot is free
+                if (e == hipSuccess) e = copy(n);
                 continue;
             }
-            if (pinned_) e = hipEventSynchronize(event(taken));
-            const Chunk *c = chunk(taken);
-            if (e == hipSuccess && !up) R.out(c->r0, c->r1, slot(taken), segs[c->seg].dst);
-            ++taken;
+            e = hipStreamSynchronize(stream);
+            if (e == hipSuccess && n + workers < chunks.size()) e = copy(n + workers);
+            if (e == hipSuccess) R.out(c.r0, c.r1, slot(n), segs[c.seg].dst);
         }
         if (e != hipSuccess) (void)hipStreamSynchronize(stream);  // nothing in flight on the slots
         return e;
