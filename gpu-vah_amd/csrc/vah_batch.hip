@@ -53,13 +53,9 @@ struct Variant {
     BatchStageFn fn;
 };
 
-// Tile shapes and eta chunks the autotuner chooses from.  64 boost-invariant
-// events of side 101-261 take 0.88 / 0.91 / 0.92 ms per step with 16 x 15, 16 x 7 and
-// 8 x 7 tiles, three 3+1D events of side 121-181 2.41 / 2.38 / 2.47 with three planes
-// and, with six, 2.33 in 16 x 7 and 2.37 in 8 x 7; a few events (whose tiles do not
-// fill the chip) least with the smallest tile, which is the default.
-// Callers may have stored an index: 0 and 1 keep their tile and chunk, 2 to 5 are the
-// shapes that took the places of 32 x 7 tiles and of a third workgroup per CU.
+// Tile shapes and eta chunks the autotuner chooses from.  Callers may have stored an
+// index: 0 and 1 keep their tile and chunk, 2 to 5 are the shapes that took the places
+// of 32 x 7 tiles and of a third workgroup per CU.
 const Variant kVariants[] = {
     {{16, 15, kWavesPerSimd, 3}, 4, batch_stage_t16x15},
     {{16, 15, kWavesPerSimd, 6}, 4, batch_stage_t16x15},
@@ -68,7 +64,17 @@ const Variant kVariants[] = {
     {{8, 7, kWavesPerSimd, 3}, 1, batch_stage_t8x7},
     {{8, 7, kWavesPerSimd, 6}, 1, batch_stage_t8x7},
 };
-constexpr int kDefaultVariant = 4;
+// The default, by the cells of the live events.  Few cells: many small tiles, or they
+// do not fill the chip.  Many: the events' fields leave the caches, and the halo of a
+// tile comes from memory.  ms per step with 8 x 7 / 16 x 15 tiles: boost-invariant
+// events of side 101-261, 4 (0.21 M cells) 0.107 / 0.120, 24 (0.88 M) 0.419 / 0.423, 64
+// (2.4 M) 1.11 / 1.06, 128 (4.6 M) 2.21 / 2.02, 512 (18 M) 9.28 / 7.80; 3+1D events of
+// side 121-201, 1 (2.6 M) 1.66 / 1.64, 2 (4.9 M) 3.30 / 3.02, 16 (27 M) 20.9 / 16.6; a
+// fifth of them 3+1D, 5 (2.2 M) 1.39 / 1.53, 10 (3.9 M) 2.47 / 2.44, 40 (13 M) 9.07 /
+// 7.97.  (8 x 7 alone lost 3 % at 2,048 events to the 16 x 15 kernels before the roles.)
+// The gap between the two lines keeps a batch near one of them from going back and forth.
+constexpr int kDefaultVariant = 4, kLargeVariant = 1;
+constexpr long kLargeFrom = 4000000, kLargeDownTo = 3000000;
 constexpr int kNumVariants = (int)(sizeof kVariants / sizeof kVariants[0]);
 
 struct HostEvent {
@@ -112,6 +118,7 @@ struct vah_batch {
     int n2, n3, nactive;
     // kernels
     int variant;
+    bool variant_by_load;  // no index given: upload_lists chooses
     std::map<int, hipGraphExec_t> graphs;  // key: (has2d, has3d)
     // pinned staging buffers for admissions, reused round-robin once their
     // copies have completed
@@ -229,9 +236,43 @@ void drop_graphs(vah_batch *b) {
     b->graphs.clear();
 }
 
+// Changes the kernels of a batch: waits for the steps that use the old ones, and
+// rewrites the descriptors, which hold the tile counts.
+int use_variant(vah_batch *b, int index) {
+    HIP_TRY(hipStreamSynchronize(b->stream));
+    drop_graphs(b);
+    b->variant = index;
+    b->lists_dirty = true;
+    std::vector<BatchEvent> desc;
+    for (int s = 0; s < b->max_events; ++s) {
+        HostEvent &h = b->events[s];
+        if (!h.used) continue;
+        fill_descriptor(b, h);
+        desc.resize(s + 1);
+        desc[s] = h.dev;
+    }
+    if (desc.empty()) return VAH_OK;
+    HIP_TRY(hipMemcpyAsync(b->ev_dev, desc.data(), sizeof(BatchEvent) * desc.size(), hipMemcpyHostToDevice, b->stream));
+    HIP_TRY(hipStreamSynchronize(b->stream));
+    return VAH_OK;
+}
+
+// the default for the events that are live now
+int variant_for_load(const vah_batch *b) {
+    long cells = 0;
+    for (const HostEvent &h : b->events)
+        if (h.used && !h.stopped) cells += h.lay.interior();
+    return cells >= (b->variant == kLargeVariant ? kLargeDownTo : kLargeFrom) ? kLargeVariant : kDefaultVariant;
+}
+
 // rebuild and upload the tile and slot lists (the stream is idle or the
 // uploads are ordered after the work that reads the old lists)
 int upload_lists(vah_batch *b) {
+    if (b->variant_by_load) {
+        const int v = variant_for_load(b);
+        int rc;
+        if (v != b->variant && (rc = use_variant(b, v)) != VAH_OK) return rc;
+    }
     std::vector<int2> t2, t3;
     std::vector<int> act, ev3;
     for (int s = 0; s < b->max_events; ++s) {
@@ -507,6 +548,7 @@ int vah_batch_create(const vah_batch_options *opt_in, vah_batch **out) {
     b->max_events = opt.max_events;
     b->events.resize(opt.max_events);
     b->variant = opt.variant < 0 ? kDefaultVariant : opt.variant;
+    b->variant_by_load = opt.variant < 0;
     b->lists_dirty = true;
     auto cleanup = [&](int code) {
         vah_batch_destroy(b);
@@ -872,20 +914,10 @@ int vah_batch_memory(const vah_batch *b, size_t *used, size_t *budget) {
 
 int vah_batch_set_variant(vah_batch *b, int index) {
     if (!b || index < 0 || index >= kNumVariants) return fail(VAH_ERR_ARG, "vah_batch_set_variant: bad variant");
+    b->variant_by_load = false;
     if (index == b->variant) return VAH_OK;
     HIP_TRY(hipSetDevice(b->device));
-    HIP_TRY(hipStreamSynchronize(b->stream));
-    drop_graphs(b);
-    b->variant = index;
-    for (int s = 0; s < b->max_events; ++s) {
-        HostEvent &h = b->events[s];
-        if (!h.used) continue;
-        fill_descriptor(b, h);
-        HIP_TRY(hipMemcpyAsync(b->ev_dev + s, &h.dev, sizeof(BatchEvent), hipMemcpyHostToDevice, b->stream));
-        HIP_TRY(hipStreamSynchronize(b->stream));
-    }
-    b->lists_dirty = true;
-    return VAH_OK;
+    return use_variant(b, index);
 }
 
 int vah_batch_get_variant(const vah_batch *b) { return b ? b->variant : -1; }

@@ -54,7 +54,7 @@ typedef struct vah_batch_options {
     int max_events;            /* resident event slots */
     double freezeout_T_GeV;    /* stop an event when T(max e) falls below this; <= 0: never */
     int steps_per_graph;       /* steps captured per hipGraph launch; 0: plain launches */
-    int variant;               /* kernel variant (vah_batch_variant_info); -1: default */
+    int variant;               /* kernel variant (vah_batch_variant_info); -1: by the live events' cells */
     int device;                /* HIP device ordinal */
     void *stream;              /* hipStream_t; NULL: a library-owned stream */
 } vah_batch_options;

@@ -1,9 +1,10 @@
 """The batch engine's kernel variants (vah_batch_variant_info, vah_batch_set_variant):
 the indices that callers may have stored."""
+import numpy as np
 import pytest
 
 from tests.parity import vah
-from tests.test_gpu_batch import admit, events_mixed
+from tests.test_gpu_batch import admit, events_mixed, same
 
 ACCEPTED = 6  # indices 0 to 5 have been accepted since the first variants
 
@@ -41,3 +42,42 @@ def test_every_stored_index_is_accepted():
         V.Batch(variant=ACCEPTED, **kw)
     assert B.poll()[0]["nstep"] == 2 * ACCEPTED
     B.close()
+
+
+@pytest.mark.gpu
+def test_default_follows_the_load():
+    """Without an index, few live cells run in 8 x 7 tiles and four million or more in
+    16 x 15 until they fall below three; the fields are those of one explicit variant
+    all the way, graphs replayed before and after each change included."""
+    V = vah()
+    small = events_mixed()[0]
+    n = 2001  # 4.004 M cells
+    x = (np.arange(n) - (n - 1) / 2) * 0.1
+    e = (20.0 * np.exp(-(x[None, :] ** 2 + 2 * x[:, None] ** 2) / 2000.0) + 1.0).ravel()
+    large = dict(small, nx=n, ny=n, nz=1, e=e)
+    kw = dict(budget_bytes=V.batch_event_bytes(n, n, 1) + (1 << 28), max_events=3, freezeout_T_GeV=0.0,
+              steps_per_graph=2)
+    got = []
+    for variant in (-1, 4):
+        B = V.Batch(variant=variant, **kw)
+        shapes = []
+
+        def steps(k):
+            B.step(k)
+            tx, ty, _, kz = V.batch_variants()[B.variant]
+            shapes.append((tx, ty, kz))
+
+        a = admit(B, small)
+        steps(4)
+        b = admit(B, large)
+        steps(5)
+        states = [B.state(s) for s in (a, b)]
+        B.retire(b)
+        steps(3)
+        states.append(B.state(a))
+        got.append((shapes, states))
+        B.close()
+    assert got[0][0] == [(8, 7, 3), (16, 15, 6), (8, 7, 3)], got[0][0]
+    assert got[1][0] == [(8, 7, 3)] * 3
+    for s, t in zip(got[0][1], got[1][1]):
+        assert same(s, t)
