@@ -299,8 +299,12 @@ LaunchCfg launch_cfg(const vah_ctx *c) {
 
 template <bool S2, typename R>
 void launch(const LaunchCfg &L, const StageParams &P) {
-    hipLaunchKernelGGL((stage_kernel<false, S2, R, kTileX, kTileWaves>), dim3(L.grid), dim3(128 * kTileWaves), 0,
-                       L.stream, P);
+    if (L.wide)
+        hipLaunchKernelGGL((stage_kernel<false, S2, R, kWideTileX, kWideTileWaves>), dim3(L.grid),
+                           dim3(128 * kWideTileWaves), 0, L.stream, P);
+    else
+        hipLaunchKernelGGL((stage_kernel<false, S2, R, kTileX, kTileWaves>), dim3(L.grid), dim3(128 * kTileWaves), 0,
+                           L.stream, P);
 }
 
 template <bool S2>

@@ -11,7 +11,7 @@ constexpr int kTileX = 8;
 constexpr int kTileY = 7;
 constexpr int kTileWaves = 1;  // waves per role
 
-// Tile of the single-lattice kernels on large 3+1D lattices: 16 x 7 cells, two
+// Tile of the single-lattice kernels on large lattices: 16 x 7 cells, two
 // waves per role.  A field's row with its halo is 20 doubles, 2.2 lines of 128 bytes
 // on average, where two tiles of 8 x 7 need 1.7 each (choose_wide_tiles says where
 // that pays).
@@ -38,10 +38,18 @@ constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // 385 / 391, 121x121x50 (2,448) 473 / 457, 151x151x101 1322 / 1200, 201x201x101
 // 2267 / 2024, 301x301x31 1597 / 1398; split 101x101x60 379 / 379, 121x121x50
 // 459 / 440, 201x201x101 2243 / 1986.  Tiles of 16 x 15 (four waves per role):
-// 2238 at 201x201x101; 2+1D at 611x587: 133 / 140.
+// 2238 at 201x201x101.  On a boost-invariant lattice, whose workgroups are shorter,
+// they pay from about a million cells on, where the halo's rows come from memory: FP64
+// 611x587 137 / 136, 801x801 251 / 249, 1001x1001 (9,009 workgroups) 422 / 414 us,
+// 2001x2001 1.65 / 1.60, 3001x3001 3.63 / 3.51, 4001x4001 7.84 / 7.10 ms; split 801x801
+// 246 / 247, 1001x1001 410 / 409 us, 2001x2001 1.61 / 1.57, 4001x4001 7.82 / 7.11 ms.
+// (The kernels before the roles, of 16 x 15 tiles, took 7.12 and 6.89 ms there; with the
+// role kernels 16 x 15 tiles take 7.82 and 7.76.)
+// Narrow ones stay out, whose rows the L2 keeps until the next row of tiles needs them:
+// 129x8001 427 / 436 us, split 417 / 440; 769x1401 448 / 438, split 439 / 436.
 inline bool choose_wide_tiles(int nx, int ny, int nz) {
     const long tiles = (long)ceil_div(nx, kWideTileX) * ceil_div(ny, kTileY);
-    return nz > 1 && tiles * ceil_div(nz, 3) >= 2300;
+    return nz > 1 ? tiles * ceil_div(nz, 3) >= 2300 : tiles >= 9000 && nx >= 48 * kWideTileX;
 }
 
 // Eta planes per workgroup when the caller leaves the choice (opt.eta_chunk 0).

@@ -11,6 +11,7 @@ import pytest
 
 from tests import test_gpu_tiles
 from tests.parity import gaussian_ic, rest_frame, vah
+from tests.test_gpu_batch import admit, worst
 from tests.test_gpu_tiles import check, run
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "gpu-vah_amd", "csrc")
@@ -27,7 +28,8 @@ extern "C" void geometry(int nx, int ny, int nz, int shared, int eta_chunk, int 
 # (lattice, tiles of 16 x 7 or 8 x 7, kz)
 CHOSEN = [((17, 8, 1725), True, 3), ((17, 8, 1722), False, 3), ((17, 8, 3073), True, 6), ((17, 8, 3066), True, 3),
           ((17, 8, 766), False, 3), ((17, 8, 765), False, 2), ((17, 8, 511), False, 2), ((17, 8, 510), False, 1),
-          ((611, 587, 1), False, 1)]
+          ((611, 587, 1), False, 1), ((785, 1253, 1), False, 1), ((785, 1254, 1), True, 1),
+          ((767, 9000, 1), False, 1), ((768, 1310, 1), True, 1), ((1001, 1001, 1), True, 1)]
 
 
 @pytest.fixture(scope="module")
@@ -60,7 +62,7 @@ def test_geometry_covers_the_lattice(geometry):
         assert 1 <= g["kz"] <= dims[2] and 0 <= g["zchunks"] * g["kz"] - dims[2] < g["kz"]
         assert g["kz"] == min(chunk, dims[2]) or chunk == 0
         assert g["nblocks"] == tiles * g["zchunks"] and g["grid"] == g["zchunks"] * 8 * -(-tiles // 8)
-        assert not g["wide"] or (shared and dims[2] > 1)
+        assert not g["wide"] or shared
 
 
 def test_chosen_tiles_and_chunks(geometry):
@@ -86,6 +88,35 @@ def test_gpu_tile_tests_take_the_tiles_they_name(geometry):
 def test_automatic_chunks(oracle_mod, dims, precision):
     """The chunks that the rule picks, with a last one of a single plane or two."""
     check(*run(vah(), oracle_mod, *dims, precision, 0), precision, str(dims))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "split"])
+@pytest.mark.parametrize("dims", [(785, 1254, 1), (799, 1261, 1), (768, 1310, 1)])
+def test_wide_tiles_in_two_dimensions(geometry, dims, precision):
+    """One cell over, on and under 16 and 7, against a batch of the one event in 8 x 7
+    tiles (1e-12, as every event of a batch; split 1e-4 in e and u).  Not against the
+    oracle: among a million lumpy cells some take another branch of the scheme there, by
+    1.7e-10, in 8 x 7 tiles and in the kernels before the roles just the same."""
+    assert geometry(dims)["wide"]
+    V = vah()
+    nx, ny, nz = dims
+    e = np.maximum(gaussian_ic(nx, ny, nz, dz=0.3, seed=nx + ny + nz, peak=60.0, tilt=0.2), 1.0)
+    g = V.Vah(nx, ny, nz, 0.1, 0.1, 0.3, 0.01, 0.2, 0.5, precision=precision)
+    g.set_primitives(e, *rest_frame(e.size), pl=e / 3)
+    g.step(3)
+    g.synchronize()
+    B = V.Batch(budget_bytes=V.batch_event_bytes(*dims) + (1 << 20), max_events=1, freezeout_T_GeV=0.0, variant=4,
+                precision=precision)
+    slot = admit(B, dict(nx=nx, ny=ny, nz=nz, dx=0.1, dy=0.1, dz=0.3, dt=0.01, t0=0.5, etabar=0.2, e=e))
+    B.step(3)
+    a, b, tau = g.state(), B.state(slot), B.poll()[0]["tau"]
+    g.close()
+    B.close()
+    if precision == 0:
+        assert worst(a, b, tau) <= 1e-12
+    else:
+        check(a, b, tau, precision, str(dims))
 
 
 @pytest.mark.gpu
