@@ -24,7 +24,7 @@
 // two waves per SIMD) was that of the union of both halves.
 // Measured, one step: 81x81 57 -> 20 us, 261x243 56 -> 43 us, 611x587 172 ->
 // 153 us, 101x101x30 296 -> 194 us, 97x89x33 in split precision 336 -> 180 us,
-// 201x201x101 2.55 -> 2.40 ms.
+// 201x201x101 2.55 -> 2.40 ms; with what came later 18, 37, 136, 171, 167 us, 2.01 ms.
 // VAH_FLUX_PER_CELL keeps the reference's work split in a kernel of its own:
 // every cell solves both of its faces with its own Newton guess.
 // Workgroups are mapped to tiles so that the eight XCDs work through the eta
